@@ -3,14 +3,13 @@
 // One workgroup of 256 threads (four wave64s) per (image, 16x16 tile), as in the reference
 // (splax/_rasterize/_kernels.py:63-87,469-500). Each wave owns one 8x8 quadrant of the tile and
 // each 16-lane row of a wave one 4x4 sub-block of it. The tile's sorted range is staged in LDS in
-// batches of records (three float4 per record; 256 per forward batch, 128 per backward batch).
+// batches of records (three float4 per record; 256 per forward batch, 112 per backward batch).
 // Each packed record carries
 //   - sigma_max: a conservative bound (log(255 o) + 1e-3) above which o e^-sigma < 1/255, so a
 //     lane skips the exponential for pairs the reference rejects anyway,
 // and while staging each record gets
 //   - a 16-bit sub-block mask: the 4x4 sub-blocks whose pixel centres can reach
-//     sigma <= sigma_max (the forward from the ellipse's exact extent per band of rows, the
-//     backward from its bounding box);
+//     sigma <= sigma_max (from the ellipse's exact extent per band of rows);
 // and each row then walks only the compacted, order-preserving list of records that reach its
 // sub-block (the four rows of a wave walk their own lists in lockstep, each row reading its own
 // record, an LDS broadcast within the row). A wave takes as many steps as its longest row list,
@@ -19,17 +18,16 @@
 // blended pairs (and every float operation on it) is the reference's, and the forward image is
 // bit-identical to the CPU oracle.
 //
-// Backward: the same staging walked back to front from the workgroup's largest final_idx, each
-// wave over the list of its whole quadrant (per-row walks there cost more in LDS bank conflicts
-// and same-record accumulator collisions than they save in steps). A pixel's contribution to a
-// record is nine floats; per record the contributing lanes of a wave reduce them with a
-// reduce-scatter (v_permlane32_swap, v_permlane16_swap, then bank-masked DPP adds within rows:
-// 19 VALU for nine values) and add the totals into the record's LDS accumulator. After each batch every record
-// stores its nine sums (plain stores, no global atomics) at its emission position, where all
-// intersections of one item are contiguous; grad_gather_kernel then adds them per item in a
-// fixed order and writes the four gradient outputs. The LDS sums of one record over the tile's
-// four quadrant waves take two accumulator copies, each added into by two waves, so no sum depends
-// on the order in which the waves arrive: the backward is deterministic.
+// Backward: the same row walks, back to front from the workgroup's largest final_idx. A step
+// leaves each pixel two numbers (its blend weight and v_sigma) of which the record wants nine
+// sums over the row's pixels; four steps at a time they are transposed over each quad of lanes,
+// so that a lane forms the sums of four pixels of one step by FMAs, and the quads' sums are
+// reduced over the row (23 VALU per step; reducing nine values per step over the wave took 27
+// VALU for a quarter of the records) and added into the wave's own LDS sums of the record. After
+// each batch every record's four waves' sums are added and stored (plain stores, no atomics
+// anywhere) at its emission position, where all intersections of one item are contiguous;
+// grad_gather_kernel then adds them per item in a fixed order and writes the four gradient
+// outputs. No sum depends on the order in which waves arrive: the backward is deterministic.
 #include <hip/hip_ext.h>
 
 #include <type_traits>
@@ -94,25 +92,16 @@ __global__ void __launch_bounds__(256) pack_records_kernel(PackParams P) {
     for (int k = threadIdx.x; k < count; k += 256) dst[k] = s_rec[k];
 }
 
-// Sub-blocks (bit 4 r + c: block row r, column c of the tile's 4x4 grid of 4x4 pixel blocks)
-// of the tile at (tile_x, tile_y) whose pixel centres a packed record can reach.
-__device__ __forceinline__ uint32_t subblock_mask(const float4& r0, const float4& r3,
-                                                  int tile_x, int tile_y) {
+// Whether a packed record can reach a pixel centre of the 8x8 quadrant whose first one is
+// (qx, qy): its box of half-widths (ex, ey) against the quadrant's. The backward's test: cheaper
+// than the forward's per-band one, and a record that reaches no pixel costs it only the sigma
+// test.
+__device__ __forceinline__ bool box_reaches(const float4& r0, const float4& r3, float qx,
+                                            float qy) {
     const uint32_t mode = __float_as_uint(r3.z);
-    if (mode == kCullNone) return 0u;
-    if (mode != kCullBox) return 0xffffu;
-    uint32_t xm = 0u, ym = 0u;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const float x0 = (float)(tile_x * kBlockWidth + c * 4) + 0.5f;
-        const float y0 = (float)(tile_y * kBlockWidth + c * 4) + 0.5f;
-        xm |= ((r0.x + r3.x >= x0) && (r0.x - r3.x <= x0 + 3.0f)) ? (1u << c) : 0u;
-        ym |= ((r0.y + r3.y >= y0) && (r0.y - r3.y <= y0 + 3.0f)) ? (1u << c) : 0u;
-    }
-    uint32_t m = 0u;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) m |= ((ym >> r) & 1u) ? (xm << (4 * r)) : 0u;
-    return m;
+    const bool box = r0.x + r3.x >= qx && r0.x - r3.x <= qx + 7.0f && r0.y + r3.y >= qy &&
+                     r0.y - r3.y <= qy + 7.0f;
+    return mode == kCullBox ? box : mode == kCullKeep;
 }
 
 // The forward's sub-block mask: the sub-blocks whose pixel centres the record can reach, from the
@@ -192,88 +181,69 @@ __device__ __forceinline__ uint32_t subblock_mask_tight(const float4& r0, const 
 }
 
 // LDS records of one batch: r0 = (x, y, a/2, b), r1 = (c/2, o, sigma_max, 1/a), r2 = (red, green,
-// blue, depth), each record's sub-block mask, and compacted record lists: with kRows (the
-// forward) one per sub-block, of record byte offsets (16 t for slot t: the address needs no
-// shift), otherwise (the backward) one per quadrant wave, of slot indices. The backward's four
-// lists (with 128-record batches and two accumulator copies) keep its LDS at 19.7 KB.
-template <bool kRows, int kBatch>
+// blue, depth), each record's sub-block mask, and one compacted record list per sub-block, of
+// record byte offsets (16 t for slot t: the address needs no shift).
+template <int kBatch>
 struct BatchLds {
     float4 r0[kBatch];
     float4 r1[kBatch];
     float4 r2[kBatch];
     uint16_t mask[kBatch];
-    // a backward wave reads its whole list row as one dword per lane: rows of kTile bytes
-    typename std::conditional<kRows, uint16_t, uint8_t>::type list[kRows ? 16 : 4][kTile];
+    __attribute__((aligned(8))) uint16_t list[16][kBatch];
 };
-// Records per batch of the backward: 128 keeps its LDS (records, lists and two accumulator
-// copies) at 19.7 KB, so with at most 64 VGPRs eight workgroups share a CU (eight waves per SIMD).
-constexpr int kBwdBatch = 128;
 
 // Stages the record of item `id` (the sorted range's entry for slot `tid`) into slot `tid` (one
-// barrier), then each wave builds its own record lists from the staged masks, in slot order:
-// with kRows the lists of its four sub-blocks (one per 16-lane row), otherwise the list of its
-// whole quadrant (a record reaches a quadrant when it reaches one of its sub-blocks, which is the
-// 8x8 box test). `live` is false for the clamped tail slots of the last batch (they reach no
-// sub-block). Returns the length of the wave's longest list, with kRows plus 65536 times the
-// calling lane's row list length.
-template <bool kRows, int kBatch>
-__device__ __forceinline__ int stage_batch(const BlendCommon& C, BatchLds<kRows, kBatch>& L,
-                                           int32_t id, bool live, int tile_x, int tile_y) {
+// barrier), then each wave builds the lists of its four sub-blocks (one per 16-lane row) from the
+// staged masks, in slot order; row r leaves out the slots below first[r]. `live` is false for the
+// clamped tail slots of the last batch (they reach no sub-block). Returns the length of the
+// wave's longest list plus 65536 times the calling lane's row list length.
+template <int kBatch, bool kFirst>
+__device__ __forceinline__ int stage_batch(const BlendCommon& C, BatchLds<kBatch>& L, int32_t id,
+                                           bool live, int tile_x, int tile_y,
+                                           const int (&first)[4], int32_t* s_clamped) {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, row = lane >> 4;
     int64_t g = id;
-    uint32_t m = 0u;
-    float4 r0 = make_float4(0.f, 0.f, 0.f, 0.f), r1 = r0, r2 = r0;
-    if (live && g >= 0 && g < C.total) {
-        const float4* rec = C.recs + 4 * g;
-        r0 = rec[0];
-        r1 = rec[1];
-        r2 = rec[2];
-        m = kRows ? subblock_mask_tight(r0, r1, rec[3], tile_x, tile_y)
-                  : subblock_mask(r0, rec[3], tile_x, tile_y);
-    }
     if (kBatch == kTile || tid < kBatch) {
+        uint32_t m = 0u;
+        float4 r0 = make_float4(0.f, 0.f, 0.f, 0.f), r1 = r0, r2 = r0;
+        if (live && g >= 0 && g < C.total) {
+            const float4* rec = C.recs + 4 * g;
+            r0 = rec[0];
+            r1 = rec[1];
+            r2 = rec[2];
+            m = subblock_mask_tight(r0, r1, rec[3], tile_x, tile_y);
+        }
         L.r0[tid] = r0;
         L.r1[tid] = r1;
         L.r2[tid] = r2;
         L.mask[tid] = (uint16_t)m;
+        if constexpr (kFirst) {
+            const bool any = __ballot(r1.y > kAlphaMax) != 0ull;
+            if (lane == 0) s_clamped[wave] = any;
+        }
     }
     __syncthreads();
     // this wave's sub-blocks: rows 0..3 -> sb0, sb0 + 1, sb0 + 4, sb0 + 5
     const int sb0 = (wave >> 1) * 8 + (wave & 1) * 2;
     const uint64_t lt = (1ull << lane) - 1ull;
-    if constexpr (kRows) {
-        int n[4] = {0, 0, 0, 0};
+    int n[4] = {0, 0, 0, 0};
 #pragma unroll
-        for (int c = 0; c < (kBatch + 63) / 64; ++c) {
-            const uint32_t mc =
-                (kBatch % 64 == 0 || c * 64 + lane < kBatch) ? L.mask[c * 64 + lane] : 0u;
+    for (int c = 0; c < (kBatch + 63) / 64; ++c) {
+        const int slot = c * 64 + lane;
+        const uint32_t mc = (kBatch % 64 == 0 || slot < kBatch) ? L.mask[slot] : 0u;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int b = sb0 + (r & 1) + (r >> 1) * 4;
-                const bool bit = (mc >> b) & 1u;
-                const uint64_t bal = __ballot(bit);
-                if (bit) L.list[b][n[r] + (int)__popcll(bal & lt)] = (uint16_t)((c * 64 + lane) * 16);
-                n[r] += (int)__popcll(bal);
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-        const int mine = row == 0 ? n[0] : row == 1 ? n[1] : row == 2 ? n[2] : n[3];
-        const int a = n[0] > n[1] ? n[0] : n[1], b = n[2] > n[3] ? n[2] : n[3];
-        return (a > b ? a : b) | (mine << 16);
-    } else {
-        const uint32_t qbits = (0x33u << sb0);  // the quadrant's four sub-blocks
-        int nq = 0;
-#pragma unroll
-        for (int c = 0; c < (kBatch + 63) / 64; ++c) {
-            const bool bit = (kBatch % 64 == 0 || c * 64 + lane < kBatch) &&
-                             (L.mask[c * 64 + lane] & qbits) != 0u;
+        for (int r = 0; r < 4; ++r) {
+            const int b = sb0 + (r & 1) + (r >> 1) * 4;
+            const bool bit = ((mc >> b) & 1u) && (!kFirst || slot >= first[r]);
             const uint64_t bal = __ballot(bit);
-            if (bit) L.list[wave][nq + (int)__popcll(bal & lt)] = (uint8_t)(c * 64 + lane);
-            nq += (int)__popcll(bal);
+            if (bit) L.list[b][n[r] + (int)__popcll(bal & lt)] = (uint16_t)(slot * 16);
+            n[r] += (int)__popcll(bal);
         }
-        __builtin_amdgcn_wave_barrier();
-        return nq;
     }
+    __builtin_amdgcn_wave_barrier();
+    const int mine = row == 0 ? n[0] : row == 1 ? n[1] : row == 2 ? n[2] : n[3];
+    const int a = n[0] > n[1] ? n[0] : n[1], b = n[2] > n[3] ? n[2] : n[3];
+    return (a > b ? a : b) | (mine << 16);
 }
 
 // Wave-uniform value as a scalar (the compiler cannot prove uniformity of values derived from
@@ -343,7 +313,7 @@ struct BlendFwdParams {
 // own 79 VGPRs and six; forcing eight spills registers).
 template <bool kDepth>
 __global__ void __launch_bounds__(kTile, 7) blend_fwd_kernel(BlendFwdParams P) {
-    __shared__ BatchLds<true, kTile> L;
+    __shared__ BatchLds<kTile> L;
     const BlendCommon& C = P.c;
     const int tid = threadIdx.x;
     const int32_t tile_g = C.order[blockIdx.x];
@@ -373,8 +343,9 @@ __global__ void __launch_bounds__(kTile, 7) blend_fwd_kernel(BlendFwdParams P) {
         if (__syncthreads_count(done) >= kTile) break;
         const int32_t batch_start = range_start + bt * kTile;
         const int32_t src = iminw(batch_start + tid, range_end - 1);
-        const int lens = stage_batch<true, kTile>(C, L, C.ids[src], batch_start + tid < range_end,
-                                                  tile_x, tile_y);
+        const int lens = stage_batch<kTile, false>(C, L, C.ids[src],
+                                                   batch_start + tid < range_end, tile_x, tile_y,
+                                                   {0, 0, 0, 0}, nullptr);
         if (__ballot(!done) == 0ull) continue;
         const int wave_max = lens & 0xffff, my_len = lens >> 16;  // my_len uniform per row
         const uint16_t* list = L.list[sb];
@@ -628,82 +599,139 @@ __device__ __forceinline__ float swap16_add(float a, float b) {
                                               false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
-// keep + the `send` value of the lane that DPP control kCtrl names (all lanes valid).
-template <int kCtrl>
-__device__ __forceinline__ float dpp_pair_add(float keep, float send) {
-    const int r = __builtin_amdgcn_update_dpp(0, __float_as_int(send), kCtrl, 0xf, 0xf, false);
-    return keep + __int_as_float(r);
+// The value of lane kLane of the caller's quad (a DPP operand of the instruction that uses it).
+template <int kLane>
+__device__ __forceinline__ float quad_lane(float x) {
+    constexpr int kCtrl = kLane * 0x55;  // quad_perm [kLane, kLane, kLane, kLane]
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(0, __float_as_int(x), kCtrl, 0xf, 0xf, false));
+}
+struct QuadBlock { float v[4]; };
+
+// Sum over the quad's lanes i of lane i's x times f.v[i], for three x: one v_fmac_f32_dpp per
+// term (the compiler keeps the FMA and its DPP move apart, two VALU more per term).
+#define SPLAT_QUAD_DOT(o, x)                                                                  \
+    "v_mul_f32_dpp %[" o "], %[" x "], %[f0] quad_perm:[0,0,0,0] row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f32_dpp %[" o "], %[" x "], %[f1] quad_perm:[1,1,1,1] row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f32_dpp %[" o "], %[" x "], %[f2] quad_perm:[2,2,2,2] row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f32_dpp %[" o "], %[" x "], %[f3] quad_perm:[3,3,3,3] row_mask:0xf bank_mask:0xf\n\t"
+__device__ __forceinline__ void quad_dot3(const QuadBlock& f, float x0, float x1, float x2,
+                                          float& o0, float& o1, float& o2) {
+    asm("s_nop 1\n\t" SPLAT_QUAD_DOT("o0", "x0") SPLAT_QUAD_DOT("o1", "x1")
+            SPLAT_QUAD_DOT("o2", "x2")
+        : [o0] "=&v"(o0), [o1] "=&v"(o1), [o2] "=&v"(o2)
+        : [x0] "v"(x0), [x1] "v"(x1), [x2] "v"(x2), [f0] "v"(f.v[0]), [f1] "v"(f.v[1]),
+          [f2] "v"(f.v[2]), [f3] "v"(f.v[3]));
+}
+__device__ __forceinline__ float quad_dot(const QuadBlock& f, float x0) {
+    float o0;
+    asm("s_nop 1\n\t" SPLAT_QUAD_DOT("o0", "x0")
+        : [o0] "=&v"(o0)
+        : [x0] "v"(x0), [f0] "v"(f.v[0]), [f1] "v"(f.v[1]), [f2] "v"(f.v[2]), [f3] "v"(f.v[3]));
+    return o0;
+}
+#undef SPLAT_QUAD_DOT
+
+// Transposes two 4x4 blocks over every quad of lanes: on entry register i of a block holds event
+// i at the lane's own pixel, on exit lane q holds event q, register i at pixel i of the quad.
+// Two exchange steps (lane bit 0, then bit 1), each one v_cndmask_b32_dpp per register: 16 VALU
+// for both blocks. The compiler keeps the select and its DPP move apart (32 VALU), so the steps
+// are written here; no DPP operand was written by either of the two VALU before it (the first
+// read waits).
+__device__ __forceinline__ void quad_transpose2(QuadBlock& f, QuadBlock& s) {
+    float a0, a1, a2, a3, b0, b1, b2, b3;
+    asm("s_mov_b32 vcc_lo, 0x55555555\n\t"  // even lanes
+        "s_mov_b32 vcc_hi, 0x55555555\n\t"
+        "s_nop 1\n\t"
+        "v_cndmask_b32_dpp %[a0], %[f1], %[f0], vcc quad_perm:[0,0,2,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[a2], %[f3], %[f2], vcc quad_perm:[0,0,2,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[b0], %[s1], %[s0], vcc quad_perm:[0,0,2,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[b2], %[s3], %[s2], vcc quad_perm:[0,0,2,2] row_mask:0xf bank_mask:0xf\n\t"
+        "s_not_b64 vcc, vcc\n\t"
+        "v_cndmask_b32_dpp %[a1], %[f0], %[f1], vcc quad_perm:[1,1,3,3] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[a3], %[f2], %[f3], vcc quad_perm:[1,1,3,3] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[b1], %[s0], %[s1], vcc quad_perm:[1,1,3,3] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[b3], %[s2], %[s3], vcc quad_perm:[1,1,3,3] row_mask:0xf bank_mask:0xf\n\t"
+        "s_mov_b32 vcc_lo, 0x33333333\n\t"  // lanes 0 and 1 of each quad
+        "s_mov_b32 vcc_hi, 0x33333333\n\t"
+        "v_cndmask_b32_dpp %[f0], %[a2], %[a0], vcc quad_perm:[0,1,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[f1], %[a3], %[a1], vcc quad_perm:[0,1,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[s0], %[b2], %[b0], vcc quad_perm:[0,1,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[s1], %[b3], %[b1], vcc quad_perm:[0,1,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "s_not_b64 vcc, vcc\n\t"
+        "v_cndmask_b32_dpp %[f2], %[a0], %[a2], vcc quad_perm:[2,3,2,3] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[f3], %[a1], %[a3], vcc quad_perm:[2,3,2,3] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[s2], %[b0], %[b2], vcc quad_perm:[2,3,2,3] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %[s3], %[b1], %[b3], vcc quad_perm:[2,3,2,3] row_mask:0xf bank_mask:0xf"
+        : [a0] "=&v"(a0), [a1] "=&v"(a1), [a2] "=&v"(a2), [a3] "=&v"(a3), [b0] "=&v"(b0),
+          [b1] "=&v"(b1), [b2] "=&v"(b2), [b3] "=&v"(b3), [f0] "+v"(f.v[0]), [f1] "+v"(f.v[1]),
+          [f2] "+v"(f.v[2]), [f3] "+v"(f.v[3]), [s0] "+v"(s.v[0]), [s1] "+v"(s.v[1]),
+          [s2] "+v"(s.v[2]), [s3] "+v"(s.v[3])
+        :
+        : "vcc", "scc");
 }
 
-// x + x[row_mirror] (lane l of each 16-lane row with lane 15 - l) written only into the lanes
-// of the 4-lane banks kBanks of each row, d kept in the others: one v_add_f32_dpp with a bank
-// mask, where a select of what to keep and what to send plus the add take three VALU. The
-// compiler does not form the bank-masked add from the DPP builtins, so it is written here, with
-// the two wait states a DPP read of a VGPR written by the previous VALU instruction needs.
-template <int kBanks>
-__device__ __forceinline__ float dpp_add_mirror_banks(float d, float x) {
-    static_assert(kBanks == 0x3 || kBanks == 0xc, "banks 0-1 or 2-3");
-    if constexpr (kBanks == 0x3)
-        asm("s_nop 1\n\tv_add_f32_dpp %0, %1, %1 row_mirror row_mask:0xf bank_mask:0x3"
-            : "+v"(d) : "v"(x));
-    else
-        asm("s_nop 1\n\tv_add_f32_dpp %0, %1, %1 row_mirror row_mask:0xf bank_mask:0xc"
-            : "+v"(d) : "v"(x));
-    return d;
+// Sums eight values over the four quads of each 16-lane row, lane q of a quad kept apart from
+// the others: o1 holds the sums of g0, g2, g1, g3 in the row's banks 0..3 (four lanes each) and o2
+// those of g4, g6, g5, g7. Lane l adds lane l ^ 8 (row_ror:8; the first of a pair in the lower
+// half, the second in the upper), then l + 4 (row_shl:4, banks 0 and 2) or l - 4 (row_shr:4,
+// banks 1 and 3): bank-masked adds, which the compiler does not form (it takes a select and an
+// add for each), with the wait states that a DPP read of a VGPR written by one of the two VALU
+// before it needs.
+__device__ __forceinline__ void row_quad_sum8(float g0, float g1, float g2, float g3, float g4,
+                                              float g5, float g6, float g7, float& o1,
+                                              float& o2) {
+    float p, q, u, v;
+    asm("s_nop 1\n\t"
+        "v_add_f32_dpp %[p], %[g0], %[g0] row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %[q], %[g2], %[g2] row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %[p], %[g1], %[g1] row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %[q], %[g3], %[g3] row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %[u], %[g4], %[g4] row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %[v], %[g6], %[g6] row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+        "v_add_f32_dpp %[u], %[g5], %[g5] row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %[v], %[g7], %[g7] row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+        "v_add_f32_dpp %[o1], %[p], %[p] row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %[o1], %[q], %[q] row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+        "v_add_f32_dpp %[o2], %[u], %[u] row_shl:4 row_mask:0xf bank_mask:0x5\n\t"
+        "v_add_f32_dpp %[o2], %[v], %[v] row_shr:4 row_mask:0xf bank_mask:0xa"
+        : [p] "=&v"(p), [q] "=&v"(q), [u] "=&v"(u), [v] "=&v"(v), [o1] "=&v"(o1), [o2] "=&v"(o2)
+        : [g0] "v"(g0), [g1] "v"(g1), [g2] "v"(g2), [g3] "v"(g3), [g4] "v"(g4), [g5] "v"(g5),
+          [g6] "v"(g6), [g7] "v"(g7));
 }
-// The same with row_half_mirror (lane j of each 8-lane half with lane 7 - j): banks 0 and 2
-// (kBanks 0x5) or 1 and 3 (0xa).
-template <int kBanks>
-__device__ __forceinline__ float dpp_add_half_mirror_banks(float d, float x) {
-    static_assert(kBanks == 0x5 || kBanks == 0xa, "banks 0 and 2 or 1 and 3");
-    if constexpr (kBanks == 0x5)
-        asm("s_nop 1\n\tv_add_f32_dpp %0, %1, %1 row_half_mirror row_mask:0xf bank_mask:0x5"
-            : "+v"(d) : "v"(x));
-    else
-        asm("s_nop 1\n\tv_add_f32_dpp %0, %1, %1 row_half_mirror row_mask:0xf bank_mask:0xa"
-            : "+v"(d) : "v"(x));
-    return d;
-}
-
-// Reduce-scatter of three values over each 16-lane row. Lane l pairs with 15 - l (row_mirror):
-// the lower half sums a and the upper half b, and c is summed on its own; then lane j of each
-// 8-lane half pairs with 7 - j (row_half_mirror), the lower quad summing the a/b partial and the
-// upper one c; two quad butterflies finish. Lanes 0-3 of the row then hold the row sum of a,
-// lanes 8-11 that of b, lanes 4-7 and 12-15 that of c: seven VALU (the halves' different sums
-// are bank-masked DPP adds), where four DPP steps per value take twelve and leave three values to
-// add into LDS.
-__device__ __forceinline__ float row_reduce_scatter3(float a, float b, float c) {
-    float r = dpp_add_mirror_banks<0x3>(a, a);  // lanes 0-7: a + a[15 - l]
-    r = dpp_add_mirror_banks<0xc>(r, b);        // lanes 8-15: b + b[15 - l]
-    c = dpp_pair_add<0x140>(c, c);              // row_mirror
-    float s = dpp_add_half_mirror_banks<0x5>(r, r);  // lanes 0-3, 8-11: the a / b partials
-    s = dpp_add_half_mirror_banks<0xa>(s, c);        // lanes 4-7, 12-15: the c partials
-    s = dpp_pair_add<0xb1>(s, s);  // quad_perm [1, 0, 3, 2]
-    s = dpp_pair_add<0x4e>(s, s);  // quad_perm [2, 3, 0, 1]
-    return s;
+// The same for one value: its sum in banks 0 and 2.
+__device__ __forceinline__ float row_quad_sum(float g) {
+    float w, o;
+    asm("s_nop 1\n\t"
+        "v_add_f32_dpp %[w], %[g], %[g] row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_add_f32_dpp %[o], %[w], %[w] row_shl:4 row_mask:0xf bank_mask:0x5"
+        : [w] "=&v"(w), [o] "=&v"(o)
+        : [g] "v"(g));
+    return o;
 }
 
-// Record accumulator slot k of batch record t, copy c ([t][c][kAccSlots] layout: the lanes that
-// add at once hit different banks). Slots 0-7 hold g0..g7; slots 8-11 hold per-row partials of
-// the last sums, which the batch readout adds: g8 from each of the four rows, or with the depth
-// channel g8 from rows 0-1 and g9 from rows 2-3. Waves 0 and 1 add into copy 0, waves 2 and 3
-// into copy 1, so a slot receives at most two adds into its zero: 0 + a + b rounds as 0 + b + a
-// (float addition commutes), whatever order the waves arrive in, and the readout adds copy 0 and
-// copy 1 in that order. Every sum is therefore the same from run to run.
-constexpr int kAccSlots = 12;
-constexpr int kAccCopies = 2;
-constexpr int kAccStride = kAccSlots * kAccCopies;
-#define ACC(t, k) acc[(t) * kAccStride + (k)]
+// The backward is bound by VALU issue. Its walk unit is the row and its record sums are one LDS
+// copy per wave: a wave-uniform walk over the quadrant's list (one record for 64 pixels, of which
+// 20 blend it) with two shared copies and ds_add_f32 took 279M VALU instructions and kept the LDS
+// busy for 0.83 of 485 us (1M gaussians at 1920x1080, under counters; 1789 us for 16 512x512
+// images of 500K); this one takes 200M in 347 us (1250 us), the LDS busy for 0.52.
+// 112 records per batch (a multiple of 16, for whole list words) keep the LDS at 25.9 KB, six
+// workgroups per CU with at most 80 VGPRs; 64, 80, 96 and 128 (five workgroups) were 1 to 4%
+// slower over the whole step. The sums of a wave are acc[wave][k][slot], kBwdStride slots apart:
+// the four k that one read takes lie 52 banks apart.
+constexpr int kBwdBatch = 112;
+constexpr int kBwdStride = 116;
 
 // kDepth adds the depth channel of _rasterize_bwd_depth_kernel / _blend_depth_vjp
 // (splax/_rasterize/_kernels.py:935-1080,1257-1302): the record's depth joins the colour dot
 // product (v_alpha and the accumulator), and v_depth = v_out_depth * fac is a tenth sum.
 template <bool kDepth>
-__global__ void __launch_bounds__(kTile, 8) blend_bwd_kernel(BlendBwdParams P) {
+__global__ void __launch_bounds__(kTile, kDepth ? 5 : 6) blend_bwd_kernel(BlendBwdParams P) {
     constexpr int NG = kDepth ? 10 : 9;
-    __shared__ BatchLds<false, kBwdBatch> L;
-    __shared__ float acc[kBwdBatch * kAccStride];
-    __shared__ int32_t s_max;
+    __shared__ BatchLds<kBwdBatch> L;
+    __shared__ float acc[4][NG][kBwdStride];
+    __shared__ int32_t s_max, s_clamped[2];
 
     const BlendCommon& C = P.c;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -771,15 +799,21 @@ __global__ void __launch_bounds__(kTile, 8) blend_bwd_kernel(BlendBwdParams P) {
     // running sum
     float acc_v = tfbg;
     if (tid == 0) s_max = range_start - 1;
-    for (int k = tid; k < kBwdBatch * kAccStride; k += kTile) acc[k] = 0.0f;
+    for (int k = tid; k < 4 * NG * kBwdStride; k += kTile) (&acc[0][0][0])[k] = 0.0f;
     __syncthreads();
     atomicMax(&s_max, bin_final);
-    // wave-wide largest final index: a record above it has no contributing lane in this wave
-    // (a DPP maximum into lane 63 with the sign bit flipped, so the unsigned order is the signed
-    // one; every lane is active here)
-    const uint32_t wm = wave_minmax_to_lane63<true>((uint32_t)bin_final ^ 0x80000000u);
-    const int32_t wmax =
-        (int32_t)((uint32_t)__builtin_amdgcn_readlane((int)wm, 63) ^ 0x80000000u);
+    // each row's largest final index: a record above it has no contributing lane there (a DPP
+    // maximum into the row's last lane with the sign bit flipped, so the unsigned order is the
+    // signed one; every lane is active here)
+    uint32_t rm = (uint32_t)bin_final ^ 0x80000000u;
+    rm = dpp_minmax_step<true, 0x111, 0xf>(rm);  // row_shr:1
+    rm = dpp_minmax_step<true, 0x112, 0xf>(rm);  // row_shr:2
+    rm = dpp_minmax_step<true, 0x114, 0xf>(rm);  // row_shr:4
+    rm = dpp_minmax_step<true, 0x118, 0xf>(rm);  // row_shr:8
+    int32_t rmax[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        rmax[r] = (int32_t)((uint32_t)__builtin_amdgcn_readlane((int)rm, 16 * r + 15) ^ 0x80000000u);
     __syncthreads();
     // a final_idx from the matching forward lies inside the tile's range; clamp anything else
     const int32_t start_idx = iminw(s_max, range_end - 1);
@@ -796,16 +830,21 @@ __global__ void __launch_bounds__(kTile, 8) blend_bwd_kernel(BlendBwdParams P) {
         }
     }
 
-    const int row = lane >> 4, l16 = lane & 15;
-    // After the wave reduction below, lane 0 of row r holds the sum of g[ka], lane 8 that of
-    // g[4 + ka] and lane 4 the row's partial for slot 8 + r; they alone add into LDS.
-    const int ka = (row == 0) ? 0 : (row == 1) ? 2 : (row == 2) ? 1 : 3;
-    const bool adds = l16 == 0 || l16 == 4 || l16 == 8;
-    const int kslot = (l16 == 0 ? ka : l16 == 8 ? 4 + ka : 8 + row) + kAccSlots * (wave >> 1);
+    const int row = lane >> 4, bank = (lane >> 2) & 3, quad_lane_id = lane & 3;
+    const int sb = row_subblock(tid);
+    // After a group's reduction lane q of bank b of a row holds event q's sums of g[kb] and
+    // g[4 + kb], and of bank 0 that of g8 (and g9).
+    const int kb = bank == 0 ? 0 : bank == 1 ? 2 : bank == 2 ? 1 : 3;
+    char* const my_acc = reinterpret_cast<char*>(&acc[wave][kb][0]);
+    const uint32_t off_sel = 0x0c0c0000u | (uint32_t)((2 * quad_lane_id + 1) << 8 | 2 * quad_lane_id);
+    const char* const rec_base = reinterpret_cast<const char*>(L.r0);
+    // blend_exp's constants that enter as addends, held in registers
+    float exp_round = 0x1.8p23f, exp_c5 = kBlendExpC5;
+    asm volatile("" : "+v"(exp_round), "+v"(exp_c5));
+    // the list words past a list's end are read (and unused): offsets inside the records
+    for (int k = tid; k < 16 * kBwdBatch; k += kTile) (&L.list[0][0])[k] = 0;
     // The sorted id and emission position of each batch slot are loaded one batch ahead, so a
-    // batch's staging waits on its records only, not on the ids that name them (the backward
-    // 0.431 -> 0.425 ms at config 2, 2.084 -> 2.064 at config 4; the same in the forward blend
-    // measured slower, 0.846 -> 0.858 ms at config 4).
+    // batch's staging waits on its records only, not on the ids that name them.
     int32_t next_id = 0, next_pos = -1;
     if (num_batches > 0 && tid < kBwdBatch) {
         const int32_t src0 = imaxw(start_idx - tid, range_start);
@@ -822,103 +861,130 @@ __global__ void __launch_bounds__(kTile, 8) blend_bwd_kernel(BlendBwdParams P) {
             next_id = C.ids[nsrc];
             next_pos = batch_end - kBwdBatch - tid >= range_start ? P.pos[nsrc] : -1;
         }
-        const int len = uniform(stage_batch<false, kBwdBatch>(C, L, id, live, tile_x, tile_y));
-        // the wave's list in one register: lane l holds entries 4l .. 4l + 3
-        const uint32_t list4 = reinterpret_cast<const uint32_t*>(L.list[uniform(wave)])[lane];
-        uint32_t word = 0;
-        for (int k = 0; k < len; ++k) {
-            if ((k & 3) == 0) word = __builtin_amdgcn_readlane(list4, k >> 2);
-            const int t = (int)((word >> (8 * (k & 3))) & 255u);
-            const int32_t idx = batch_end - t;
-            if (idx > wmax) continue;  // wave-uniform
-            const float4 r0 = L.r0[t], r1 = L.r1[t], r2 = L.r2[t];
-            // the whole record in the first reads (full-width reads, one address)
-            asm volatile("" ::"v"(r1.y), "v"(r2.x), "v"(r2.y), "v"(r2.z), "v"(r2.w));
-            const float dx = r0.x - px, dy = r0.y - py;
-            const float sigma = blend_sigma(r0, r1, dx, dy);
-            // bitwise: no short-circuit branch around the sigma_max read
-            const bool in_range = (idx <= bin_final) & sigma_in_range(sigma, r1.z);
-            if (__builtin_amdgcn_ballot_w64(in_range) == 0ull) continue;
-            // Every lane computes and the lanes outside the accepted set are masked by selects
-            // (an exec-masked instruction costs the same issue slot), so the wave reduction
-            // below always sees exact zeros there and no branch is needed.
-            const float vis = blend_exp(-sigma);
-            const float ov = r1.y * vis;
-            const float alpha_c = fminf(kAlphaMax, ov);  // as in the forward
-            const bool valid = in_range && alpha_c >= kAlphaThresh;
-            // a lane outside the accepted set blends alpha = 0 (a select, so whatever vis is):
-            // T / (1 - 0) = T and its weight alpha T is zero, so T and the running sum need no
-            // select of their own
-            const float alpha = valid ? alpha_c : 0.0f;
-            const float d = 1.0f - alpha;
-            float ra = __builtin_amdgcn_rcpf(d);
-            ra = fmaf(ra, fmaf(-d, ra, 1.0f), ra);
-            T = T * ra;
-            const float fac = alpha * T;
-            float cv = fmaf(r2.x, v0, fmaf(r2.y, v1, r2.z * v2));
-            if constexpr (kDepth) cv = fmaf(r2.w, vd, cv);  // depth as a fourth channel
-            const float v_alpha = fmaf(T, cv, -ra * acc_v);  // halved
-            acc_v = fmaf(cv, fac, acc_v);
-            const bool geo = valid && ov <= kAlphaMax;
-            // selects, not products with a masked zero: outside the accepted set vis and ov may be
-            // inf or NaN (blend_exp is defined for sigma <= kBlendSigmaCap only)
-            const float vs = geo ? -ov * v_alpha : 0.0f;  // v_sigma, halved
-            const float hx = vs * dx, hy = vs * dy;
-            const float g0 = v0 * fac, g1 = v1 * fac, g2 = v2 * fac;
-            const float g3 = hx * dx, g4 = hx * dy, g5 = hy * dy;  // g3, g5 whole
-            const float g6 = hx, g7 = hy;
-            // the opacity term vis v_alpha is -v_sigma / o with the record's o, so the sum of
-            // v_sigma is carried and the readout divides by -o once per record
-            const float g8 = vs;
-            const float g9 = kDepth ? vd * fac : 0.0f;
-            // reduce-scatter over the wave: after the swaps, row r of qa holds g0/g2/g1/g3 and
-            // of qb g4/g6/g5/g7 (rows 0..3); qc is g8 unswapped (each row reduces its own lanes)
-            // or with depth the one swap of g8 with g9 (rows 0-1 then carry g8, rows 2-3 g9).
-            // The row reduce-scatter leaves each sum in one adding lane.
-            const float p01 = swap32_add(g0, g1), p23 = swap32_add(g2, g3);
-            const float p45 = swap32_add(g4, g5), p67 = swap32_add(g6, g7);
-            const float qa = swap16_add(p01, p23), qb = swap16_add(p45, p67);
-            const float qc = kDepth ? swap32_add(g8, g9) : g8;
-            const float sum = row_reduce_scatter3(qa, qb, qc);
-            // An empty use keeps the last DPP add in this block: sunk into the branch below it
-            // would no longer fuse with its DPP move.
-            asm volatile("" ::"v"(sum));
-            if (adds) atomicAdd(&acc[t * kAccStride + kslot], sum);
-        }
+        const int first[4] = {batch_end - rmax[0], batch_end - rmax[1], batch_end - rmax[2],
+                              batch_end - rmax[3]};
+        const int lens = stage_batch<kBwdBatch, true>(C, L, id, live, tile_x, tile_y, first,
+                                                      s_clamped);
+        const bool clamped = uniform(s_clamped[0] | s_clamped[1]) != 0;
+        const int wave_max = uniform(lens & 0xffff), my_len = lens >> 16;  // uniform per row
+        const uint16_t* const list = L.list[sb];
+        const int32_t min_off = (batch_end - bin_final) * 16;  // the pixel's first record
+        auto walk = [&](auto clamp) {
+            constexpr bool kClamp = decltype(clamp)::value;
+            for (int k0 = 0; k0 < wave_max; k0 += 4) {
+                const uint2 offs = *reinterpret_cast<const uint2*>(list + k0);
+                QuadBlock f, s;
+    #pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    f.v[e] = 0.0f;
+                    s.v[e] = 0.0f;
+                    if (k0 + e < wave_max) {  // uniform
+                        const uint32_t pair = e < 2 ? offs.x : offs.y;
+                        const int off = (e & 1) ? (int)(pair >> 16) : (int)(pair & 0xffffu);
+                        const float4 r0 = *reinterpret_cast<const float4*>(rec_base + off);
+                        const float4 r1 =
+                            *reinterpret_cast<const float4*>(rec_base + off + sizeof(L.r0));
+                        const float4 r2 =
+                            *reinterpret_cast<const float4*>(rec_base + off + 2 * sizeof(L.r0));
+                        // the whole record in the first reads (full-width reads, one address)
+                        asm volatile("" ::"v"(r1.y), "v"(r2.x), "v"(r2.y), "v"(r2.z), "v"(r2.w));
+                        const float dx = r0.x - px, dy = r0.y - py;
+                        const float sigma = blend_sigma(r0, r1, dx, dy);
+                        const bool in_range = (k0 + e < my_len) & (off >= min_off) &
+                                              sigma_in_range(sigma, r1.z);
+                        const float vis = blend_exp(-sigma, exp_round, exp_c5);
+                        const float ov = r1.y * vis;
+                        // as in the forward; without a clamped record ov <= o <= kAlphaMax
+                        const float alpha_c = kClamp ? fminf(kAlphaMax, ov) : ov;
+                        const bool valid = in_range && alpha_c >= kAlphaThresh;
+                        // a lane outside the accepted set blends alpha = 0 (a select, so
+                        // whatever vis is): T / (1 - 0) = T and its weight alpha T is zero, so T
+                        // and the running sum need no select of their own
+                        const float alpha = valid ? alpha_c : 0.0f;
+                        const float d = 1.0f - alpha;
+                        float ra = __builtin_amdgcn_rcpf(d);
+                        ra = fmaf(ra, fmaf(-d, ra, 1.0f), ra);
+                        T = T * ra;
+                        const float fac = alpha * T;
+                        float cv = fmaf(r2.x, v0, fmaf(r2.y, v1, r2.z * v2));
+                        if constexpr (kDepth) cv = fmaf(r2.w, vd, cv);  // depth as a fourth channel
+                        const float v_alpha = fmaf(T, cv, -ra * acc_v);  // halved
+                        acc_v = fmaf(cv, fac, acc_v);
+                        // v_sigma, halved, zero where alpha was clamped: a select, since v_alpha
+                        // may be inf or NaN (a pixel's cotangent) where nothing is blended
+                        const bool geo = valid && (!kClamp || ov <= kAlphaMax);
+                        s.v[e] = geo ? -ov * v_alpha : 0.0f;
+                        f.v[e] = fac;
+                    }
+                }
+                // Lane q of each quad takes step q: a quad is one pixel row, so dy is one number
+                quad_transpose2(f, s);
+                const uint32_t off = __builtin_amdgcn_perm(offs.y, offs.x, off_sel);
+                const float2 xy = *reinterpret_cast<const float2*>(rec_base + off);
+                const float dx0 = xy.x - quad_lane<0>(px), dx1 = xy.x - quad_lane<1>(px);
+                const float dx2 = xy.x - quad_lane<2>(px), dx3 = xy.x - quad_lane<3>(px);
+                const float dy = xy.y - py;
+                float g0, g1, g2;  // sums of the cotangents times the weights
+                quad_dot3(f, v0, v1, v2, g0, g1, g2);
+                const float h0 = s.v[0] * dx0, h1 = s.v[1] * dx1, h2 = s.v[2] * dx2, h3 = s.v[3] * dx3;
+                const float g3 = fmaf(h3, dx3, fmaf(h2, dx2, fmaf(h1, dx1, h0 * dx0)));  // whole
+                const float g6 =
+                    fmaf(s.v[3], dx3, fmaf(s.v[2], dx2, fmaf(s.v[1], dx1, h0)));
+                // the opacity term vis v_alpha is -v_sigma / o with the record's o, so the sum
+                // of v_sigma is carried and the readout divides by -o once per record
+                const float g8 = (s.v[0] + s.v[1]) + (s.v[2] + s.v[3]);
+                const float g4 = g6 * dy, g7 = g8 * dy;
+                const float g5 = g7 * dy;  // whole
+                float o1, o2;
+                row_quad_sum8(g0, g1, g2, g3, g4, g5, g6, g7, o1, o2);
+                const float o3 = row_quad_sum(g8);
+                float o4 = 0.0f;
+                if constexpr (kDepth) o4 = row_quad_sum(quad_dot(f, vd));
+                const bool act = k0 < my_len - quad_lane_id;
+                float* const a = reinterpret_cast<float*>(my_acc + (off >> 2));
+                // Two rows may hold the same record, so the rows add in turn (the LDS serves a wave's
+                // reads and writes in order). The record sums of a wave are its own: plain reads and
+                // writes, where ds_add_f32 takes about three cycles per lane.
+    #pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (row == r && act) {
+                        const float x1 = a[0], x2 = a[4 * kBwdStride];
+                        a[0] = x1 + o1;
+                        a[4 * kBwdStride] = x2 + o2;
+                        if (bank == 0) {  // a is g0's row of sums
+                            a[8 * kBwdStride] += o3;
+                            if constexpr (kDepth) a[9 * kBwdStride] += o4;
+                        }
+                    }
+                    __builtin_amdgcn_wave_barrier();
+                    asm volatile("" ::: "memory");
+                }
+            }
+        };
+        // without a record opaque enough for its alpha to be clamped a step takes two VALU less
+        if (clamped)
+            walk(std::true_type{});
+        else
+            walk(std::false_type{});
         __syncthreads();
         if (tid < kBwdBatch) {
-            float s[NG], part[4];
+            float s[NG];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                // the halved sums doubled (the conic's a and c terms, slots 3 and 5, are whole)
-                const float v = ACC(tid, k) + ACC(tid, kAccSlots + k);
+            for (int k = 0; k < NG; ++k) {
+                // the halved sums doubled (the conic's a and c terms, 3 and 5, are whole)
+                const float v = (acc[0][k][tid] + acc[1][k][tid]) + (acc[2][k][tid] + acc[3][k][tid]);
                 s[k] = (k == 3 || k == 5) ? v : 2.0f * v;
-                ACC(tid, k) = 0.0f;
-                ACC(tid, kAccSlots + k) = 0.0f;
-            }
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                part[r] = ACC(tid, 8 + r) + ACC(tid, kAccSlots + 8 + r);
-                ACC(tid, 8 + r) = 0.0f;
-                ACC(tid, kAccSlots + 8 + r) = 0.0f;
+                for (int w = 0; w < 4; ++w) acc[w][k][tid] = 0.0f;
             }
             // v_opacity = sum vis v_alpha = -(sum v_sigma) / o (o >= 1/255 for every accepted
             // pair; a record with none sums to zero, which stays zero)
-            float vsig;
-            if constexpr (kDepth) {
-                vsig = 2.0f * (part[0] + part[1]);
-                s[9] = 2.0f * (part[2] + part[3]);
-            } else {
-                vsig = 2.0f * ((part[0] + part[1]) + (part[2] + part[3]));
-            }
-            s[8] = vsig != 0.0f ? -vsig / L.r1[tid].y : 0.0f;
+            s[8] = s[8] != 0.0f ? -s[8] / L.r1[tid].y : 0.0f;
             if (my_pos >= 0 && my_pos < P.M) store_rgrad<NG>(P.rgrad, rg_off + my_pos, s);
         }
         __syncthreads();
     }
 }
-
-#undef ACC
 
 // Per output item: sum of its intersections' partial gradients in emission order (fixed, so
 // deterministic; the conic and xy sums in double, the others in float), then
