@@ -367,6 +367,15 @@ int splat_mcmc_relocate(splat_stream_t stream, float* means3d, float* log_scales
                         int32_t n_max, float min_opacity, uint64_t seed, int32_t* source,
                         uint8_t* reset);
 
+/* splat_mcmc_relocate into arrays of the caller's (which must not overlap the inputs): the rows
+ * that splax.mcmc.relocate returns, in one pass over them. The inputs stay as they are. */
+int splat_mcmc_relocate_copy(splat_stream_t stream, const float* means3d, const float* log_scales,
+                             const float* quats, const float* logit_colors,
+                             const float* logit_opacities, int64_t num_gaussians, int32_t n_max,
+                             float min_opacity, uint64_t seed, float* out_means3d,
+                             float* out_log_scales, float* out_quats, float* out_logit_colors,
+                             float* out_logit_opacities, uint8_t* reset);
+
 /* Replaces splax.mcmc.inject_noise (splax/mcmc.py:134-169): out_means [n,3] = means3d +
  * Sigma (z sigmoid(100 (min_opacity - o)) scaler) with Sigma = R diag(exp(log_scales))^2 R^T
  * (R of the normalized wxyz quats [n,4]), o = sigmoid(logit_opacities [n]) and z three standard

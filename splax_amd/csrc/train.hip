@@ -245,7 +245,10 @@ __global__ void __launch_bounds__(256) inject_noise_kernel(NoiseParams P) {
 
 // ------------------------------------------------------------------ relocation
 
-constexpr int kRelocChunk = 4096;  // weights per workgroup of the scan (16 per thread)
+// Rows per workgroup of the relocation's scans and compactions (four per thread): at 1M rows 977
+// workgroups, about four per CU; 4096 rows gave 245, less than one.
+constexpr int kRelocChunk = 1024;
+constexpr int kRelocPer = kRelocChunk / 256;
 constexpr int kMaxBinomRows = 62;  // C(r, k) * (r - k) stays below 2^64 for r <= 62
 
 __device__ __forceinline__ float reloc_sigmoid(float x) { return 1.0f / (1.0f + det_expf(-x)); }
@@ -278,7 +281,11 @@ __device__ __forceinline__ void relocation_values(double o, int r, double& no, d
 }
 
 struct RelocParams {
-    float* means; float* log_scales; float* quats; float* colors; float* logit_opac;
+    const float* means; const float* log_scales; const float* quats; const float* colors;
+    const float* logit_opac;
+    // the relocated rows; the inputs themselves in place
+    float* out_means; float* out_log_scales; float* out_quats; float* out_colors;
+    float* out_logit_opac;
     int64_t n;
     int32_t n_max;
     float min_opacity;
@@ -310,7 +317,7 @@ __global__ void __launch_bounds__(256) reloc_partials_kernel(RelocParams P) {
     const int64_t base = (int64_t)blockIdx.x * kRelocChunk;
     uint64_t acc = 0;
 #pragma unroll
-    for (int j = 0; j < kRelocChunk / 256; ++j) {
+    for (int j = 0; j < kRelocPer; ++j) {
         const int64_t i = base + j * 256 + threadIdx.x;
         if (i < P.n) {
             acc += reloc_weight(P.logit_opac[i], P.min_opacity);
@@ -321,50 +328,65 @@ __global__ void __launch_bounds__(256) reloc_partials_kernel(RelocParams P) {
     if (threadIdx.x == 0) P.partials[blockIdx.x] = t;
 }
 
-// One workgroup: exclusive scan of the workgroup sums, total in partials[blocks].
-__global__ void __launch_bounds__(256) reloc_scan_partials_kernel(RelocParams P) {
-    __shared__ uint64_t s[256];
+// One workgroup: exclusive scan of the workgroup sums, total in partials[blocks]. A round takes
+// four consecutive sums per thread (4M rows in all): two barriers, where a 256-wide ladder took
+// sixteen for every 256 sums.
+constexpr int kRelocScanThreads = 1024;
+__global__ void __launch_bounds__(kRelocScanThreads) reloc_scan_partials_kernel(RelocParams P) {
+    __shared__ uint64_t s_wave[kRelocScanThreads / 64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     uint64_t carry = 0;
-    for (int64_t c0 = 0; c0 < P.blocks; c0 += 256) {
-        const int64_t i = c0 + threadIdx.x;
-        const uint64_t v = i < P.blocks ? P.partials[i] : 0ull;
-        s[threadIdx.x] = v;
-        __syncthreads();
-        for (int off = 1; off < 256; off <<= 1) {  // Hillis-Steele inclusive scan
-            const uint64_t add = threadIdx.x >= (unsigned)off ? s[threadIdx.x - off] : 0ull;
-            __syncthreads();
-            s[threadIdx.x] += add;
-            __syncthreads();
+    for (int64_t c0 = 0; c0 < P.blocks; c0 += 4 * kRelocScanThreads) {
+        const int64_t i = c0 + 4 * (int64_t)tid;
+        uint64_t v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = i + k < P.blocks ? P.partials[i + k] : 0ull;
+        const uint64_t own = (v[0] + v[1]) + (v[2] + v[3]);
+        uint64_t incl = own;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint64_t up = __shfl_up(incl, off, 64);
+            if (lane >= off) incl += up;
         }
-        if (i < P.blocks) P.partials[i] = carry + s[threadIdx.x] - v;
-        carry += s[255];
+        if (lane == 63) s_wave[wave] = incl;
         __syncthreads();
+        uint64_t run = carry + incl - own;
+        for (int w = 0; w < kRelocScanThreads / 64; ++w) {
+            const uint64_t x = s_wave[w];
+            run += w < wave ? x : 0ull;
+            carry += x;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (i + k < P.blocks) P.partials[i + k] = run;
+            run += v[k];
+        }
+        __syncthreads();  // s_wave is rewritten by the next round
     }
-    if (threadIdx.x == 0) P.partials[P.blocks] = carry;
+    if (tid == 0) P.partials[P.blocks] = carry;
 }
 
-// Inclusive prefix of the weights: each thread owns 16 consecutive weights. The weights are
+// Inclusive prefix of the weights: each thread owns kRelocPer consecutive weights. The weights are
 // computed from coalesced loads (thread t takes elements t, t + 256, ...) into LDS, where each
-// thread then reads its own 16 (rows padded by one word against bank conflicts), and the prefixes
-// leave the same way, so every global access is coalesced (config 4's relocation 0.066 -> 0.054
-// ms against per-thread runs read and written directly).
-constexpr int kCdfPad = 17;  // LDS words per thread row: 16 weights + 1 pad
+// thread then reads its own (rows padded by one word against bank conflicts), and the prefixes
+// leave the same way, so every global access is coalesced.
+constexpr int kCdfPad = kRelocPer + 1;  // LDS words per thread row: its weights + 1 pad
 __global__ void __launch_bounds__(256) reloc_cdf_kernel(RelocParams P) {
     __shared__ uint64_t s_w[256 * kCdfPad];
     __shared__ uint64_t s_wave[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t base = (int64_t)blockIdx.x * kRelocChunk;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
+    for (int j = 0; j < kRelocPer; ++j) {
         const int e = j * 256 + tid;  // element of the chunk
         const int64_t i = base + e;
         const uint64_t w = i < P.n ? reloc_weight(P.logit_opac[i], P.min_opacity) : 0ull;
-        s_w[(e >> 4) * kCdfPad + (e & 15)] = w;
+        s_w[(e / kRelocPer) * kCdfPad + (e % kRelocPer)] = w;
     }
     __syncthreads();
     uint64_t own = 0;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) own += s_w[tid * kCdfPad + k];
+    for (int k = 0; k < kRelocPer; ++k) own += s_w[tid * kCdfPad + k];
     // exclusive prefix of `own` over the workgroup: wave scan by shuffles, then the waves before
     uint64_t incl = own;
 #pragma unroll
@@ -378,90 +400,158 @@ __global__ void __launch_bounds__(256) reloc_cdf_kernel(RelocParams P) {
 #pragma unroll
     for (int w = 0; w < 4; ++w) run += w < wave ? s_wave[w] : 0ull;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
+    for (int k = 0; k < kRelocPer; ++k) {
         run += s_w[tid * kCdfPad + k];
         s_w[tid * kCdfPad + k] = run;
     }
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
+    for (int j = 0; j < kRelocPer; ++j) {
         const int e = j * 256 + tid;
         const int64_t i = base + e;
-        if (i < P.n) P.cdf[i] = s_w[(e >> 4) * kCdfPad + (e & 15)];
+        if (i < P.n) P.cdf[i] = s_w[(e / kRelocPer) * kCdfPad + (e % kRelocPer)];
     }
 }
 
-// Draws the source of every dead gaussian (splax/mcmc.py:107-111) and counts the draws.
-__global__ void __launch_bounds__(256) reloc_sample_kernel(RelocParams P) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= P.n) return;
-    if (!reloc_dead(P.logit_opac[i], P.min_opacity)) {
-        P.src[i] = (int32_t)i;
-        return;
-    }
-    const uint64_t total = P.partials[P.blocks];
-    int64_t s = 0;  // nothing alive: every logit is -inf and the reference's argmax gives 0
-    if (total > 0) {
-        uint32_t c[4] = {(uint32_t)i, (uint32_t)((uint64_t)i >> 32), kRelocateTag, 0u};
-        philox4x32_10(c, P.seed_lo, P.seed_hi);
-        const uint64_t r = ((uint64_t)c[0] << 32) | c[1];
-        const uint64_t u = __umul64hi(r, total);
-        int64_t lo = 0, hi = P.n - 1;  // first index with cdf > u; cdf[n-1] = total > u
-        while (lo < hi) {
-            const int64_t mid = (lo + hi) >> 1;
-            if (P.cdf[mid] > u) hi = mid; else lo = mid + 1;
+// First index of the nondecreasing cdf[lo, hi) above u, given cdf[hi - 1] > u: sixteen-way,
+// fifteen independent reads per round.
+__device__ __forceinline__ int64_t cdf_search(const uint64_t* cdf, int64_t lo, int64_t hi,
+                                              uint64_t u) {
+    while (hi - lo > 1) {
+        const int64_t step = (hi - lo + 15) >> 4;
+        int32_t below = 0;
+#pragma unroll
+        for (int k = 1; k < 16; ++k) {
+            const int64_t p = lo + k * step - 1;
+            below += cdf[p < hi - 1 ? p : hi - 1] <= u ? 1 : 0;  // cdf[hi - 1] > u
         }
-        s = lo;
+        lo += below * step;
+        hi = lo + step < hi ? lo + step : hi;
     }
-    P.src[i] = (int32_t)s;
-    atomicAdd(&P.counts[s], 1);
+    return lo;
+}
+
+// Collects the chunk's rows for which pick(i) holds into s_rows (any order) and returns their
+// number: the rare, long work that follows then fills whole waves (one row in twenty is dead in
+// early training; a thread per row left three lanes of each wave at work).
+template <typename Pick>
+__device__ __forceinline__ int collect_rows(int64_t n, int32_t* s_rows, int32_t* s_count,
+                                            Pick pick) {
+    if (threadIdx.x == 0) *s_count = 0;
+    __syncthreads();
+    const int64_t base = (int64_t)blockIdx.x * kRelocChunk;
+#pragma unroll
+    for (int j = 0; j < kRelocPer; ++j) {
+        const int64_t i = base + j * 256 + threadIdx.x;
+        if (i < n && pick(i)) s_rows[atomicAdd(s_count, 1)] = (int32_t)i;
+    }
+    __syncthreads();
+    return *s_count;
+}
+
+// Draws the source of every dead gaussian (splax/mcmc.py:107-111) and counts the draws. What bounds
+// it is the latency of the search's dependent random reads, so up to 4M rows the chunks' prefixes
+// are searched in LDS and only the chunk's 1024 entries in memory, three rounds of fifteen reads
+// (1M rows, 5% dead: 28 us by halving with a thread per row, 19 us collected and sixteen-way over
+// the whole cdf, 16 us so).
+constexpr int kRelocTop = 4096;  // chunk prefixes held in LDS
+__global__ void __launch_bounds__(256) reloc_sample_kernel(RelocParams P) {
+    __shared__ uint64_t s_top[kRelocTop];
+    __shared__ int32_t s_rows[kRelocChunk], s_count;
+    const int dead = collect_rows(P.n, s_rows, &s_count, [&](int64_t i) {
+        const bool d = reloc_dead(P.logit_opac[i], P.min_opacity);
+        if (!d) P.src[i] = (int32_t)i;
+        return d;
+    });
+    if (dead == 0) return;  // uniform
+    const uint64_t total = P.partials[P.blocks];
+    const bool top = P.blocks <= kRelocTop;
+    if (top) {
+        for (int c = threadIdx.x; c < P.blocks; c += 256) s_top[c] = P.partials[c];
+        __syncthreads();
+    }
+    for (int e = threadIdx.x; e < dead; e += 256) {
+        const int64_t i = s_rows[e];
+        int64_t s = 0;  // nothing alive: every logit is -inf and the reference's argmax gives 0
+        if (total > 0) {
+            uint32_t c[4] = {(uint32_t)i, (uint32_t)((uint64_t)i >> 32), kRelocateTag, 0u};
+            philox4x32_10(c, P.seed_lo, P.seed_hi);
+            const uint64_t r = ((uint64_t)c[0] << 32) | c[1];
+            const uint64_t u = __umul64hi(r, total);
+            int64_t lo = 0, hi = P.n;  // cdf[n - 1] = total > u
+            if (top) {  // the last chunk whose prefix is at most u: the next one's is above
+                int32_t c = 0;
+                for (int32_t half = kRelocTop / 2; half > 0; half >>= 1)
+                    if (c + half < P.blocks && s_top[c + half] <= u) c += half;
+                lo = (int64_t)c * kRelocChunk;
+                hi = lo + kRelocChunk < P.n ? lo + kRelocChunk : P.n;
+            }
+            s = cdf_search(P.cdf, lo, hi, u);
+        }
+        P.src[i] = (int32_t)s;
+        atomicAdd(&P.counts[s], 1);
+    }
 }
 
 // New (logit, log scales) of every drawn source, from its unmodified row.
 __global__ void __launch_bounds__(256) reloc_values_kernel(RelocParams P) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= P.n) return;
-    const int32_t cnt = P.counts[i];
-    if (cnt <= 0) return;
-    const int r = cnt + 1 < P.n_max ? cnt + 1 : P.n_max;  // ratio, clipped to [1, n_max]
-    const double o = (double)reloc_sigmoid(P.logit_opac[i]);
-    double no, coeff;
-    relocation_values(o, r, no, coeff);
-    const double lo_clip = (double)P.min_opacity, hi_clip = 1.0 - 0x1p-23;
-    no = no < lo_clip ? lo_clip : no;
-    no = no > hi_clip ? hi_clip : no;
-    float4 v;
-    v.x = (float)log(no / (1.0 - no));
-    v.y = (float)log(coeff * (double)det_expf(P.log_scales[3 * i]));
-    v.z = (float)log(coeff * (double)det_expf(P.log_scales[3 * i + 1]));
-    v.w = (float)log(coeff * (double)det_expf(P.log_scales[3 * i + 2]));
-    P.newv[i] = v;
+    __shared__ int32_t s_rows[kRelocChunk], s_count;
+    const int drawn =
+        collect_rows(P.n, s_rows, &s_count, [&](int64_t i) { return P.counts[i] > 0; });
+    for (int e = threadIdx.x; e < drawn; e += 256) {
+        const int64_t i = s_rows[e];
+        const int32_t cnt = P.counts[i];
+        const int r = cnt + 1 < P.n_max ? cnt + 1 : P.n_max;  // ratio, clipped to [1, n_max]
+        const double o = (double)reloc_sigmoid(P.logit_opac[i]);
+        double no, coeff;
+        relocation_values(o, r, no, coeff);
+        const double lo_clip = (double)P.min_opacity, hi_clip = 1.0 - 0x1p-23;
+        no = no < lo_clip ? lo_clip : no;
+        no = no > hi_clip ? hi_clip : no;
+        float4 v;
+        v.x = (float)log(no / (1.0 - no));
+        v.y = (float)log(coeff * (double)det_expf(P.log_scales[3 * i]));
+        v.z = (float)log(coeff * (double)det_expf(P.log_scales[3 * i + 1]));
+        v.w = (float)log(coeff * (double)det_expf(P.log_scales[3 * i + 2]));
+        P.newv[i] = v;
+    }
 }
 
 // Writes the relocated rows (splax/mcmc.py:119-131). Dead rows copy mean, quaternion and colour
 // of their source, which is alive and keeps those, and take the source's new values.
+// kCopy: the relocated rows go to arrays of their own and every row is written (112 bytes read
+// and written per row once, where copies of the five arrays and the in-place pass over them take
+// two passes); otherwise only the relocated rows are.
+template <bool kCopy>
 __global__ void __launch_bounds__(256) reloc_apply_kernel(RelocParams P) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= P.n) return;
     const int32_t s = P.src[i];
-    const bool dead = reloc_dead(P.logit_opac[i], P.min_opacity);  // own row, read before writing
+    const float logit = P.logit_opac[i];  // own row, read before writing
+    const bool dead = reloc_dead(logit, P.min_opacity);
     const bool reset = dead || P.counts[i] > 0;
-    if (dead) {
-        const float m0 = P.means[3 * s], m1 = P.means[3 * s + 1], m2 = P.means[3 * s + 2];
-        const float q0 = P.quats[4 * s], q1 = P.quats[4 * s + 1], q2 = P.quats[4 * s + 2],
-                    q3 = P.quats[4 * s + 3];
-        const float c0 = P.colors[3 * s], c1 = P.colors[3 * s + 1], c2 = P.colors[3 * s + 2];
-        P.means[3 * i] = m0; P.means[3 * i + 1] = m1; P.means[3 * i + 2] = m2;
-        P.quats[4 * i] = q0; P.quats[4 * i + 1] = q1; P.quats[4 * i + 2] = q2;
-        P.quats[4 * i + 3] = q3;
-        P.colors[3 * i] = c0; P.colors[3 * i + 1] = c1; P.colors[3 * i + 2] = c2;
+    if (kCopy || dead) {
+        const int64_t f = dead ? s : i;
+        const float m0 = P.means[3 * f], m1 = P.means[3 * f + 1], m2 = P.means[3 * f + 2];
+        const float q0 = P.quats[4 * f], q1 = P.quats[4 * f + 1], q2 = P.quats[4 * f + 2],
+                    q3 = P.quats[4 * f + 3];
+        const float c0 = P.colors[3 * f], c1 = P.colors[3 * f + 1], c2 = P.colors[3 * f + 2];
+        P.out_means[3 * i] = m0; P.out_means[3 * i + 1] = m1; P.out_means[3 * i + 2] = m2;
+        P.out_quats[4 * i] = q0; P.out_quats[4 * i + 1] = q1; P.out_quats[4 * i + 2] = q2;
+        P.out_quats[4 * i + 3] = q3;
+        P.out_colors[3 * i] = c0; P.out_colors[3 * i + 1] = c1; P.out_colors[3 * i + 2] = c2;
     }
-    if (reset) {
-        const float4 v = P.newv[dead ? s : (int32_t)i];
-        P.logit_opac[i] = v.x;
-        P.log_scales[3 * i] = v.y;
-        P.log_scales[3 * i + 1] = v.z;
-        P.log_scales[3 * i + 2] = v.w;
+    if (kCopy || reset) {
+        float4 v;
+        if (reset)
+            v = P.newv[dead ? s : (int32_t)i];
+        else
+            v = make_float4(logit, P.log_scales[3 * i], P.log_scales[3 * i + 1],
+                            P.log_scales[3 * i + 2]);
+        P.out_logit_opac[i] = v.x;
+        P.out_log_scales[3 * i] = v.y;
+        P.out_log_scales[3 * i + 1] = v.z;
+        P.out_log_scales[3 * i + 2] = v.w;
     }
     if (P.source_out) P.source_out[i] = s;
     if (P.reset_out) P.reset_out[i] = reset ? 1 : 0;
@@ -622,51 +712,75 @@ int splat_adam_reset_rows(splat_stream_t stream, const splat_adam_group* groups,
     return launched("adam_reset_rows");
 }
 
-int splat_mcmc_relocate(splat_stream_t stream, float* means3d, float* log_scales, float* quats,
-                        float* logit_colors, float* logit_opacities, int64_t num_gaussians,
-                        int32_t n_max, float min_opacity, uint64_t seed, int32_t* source,
-                        uint8_t* reset) {
-    if (num_gaussians < 0 || num_gaussians > 0x7fffffff)
+static int relocate_impl(splat_stream_t stream, RelocParams P, bool copy, uint64_t seed) {
+    if (P.n < 0 || P.n > 0x7fffffff)
         return fail(kErrArgs, "relocate: gaussian count outside [0, 2^31)");
-    if (n_max < 1 || n_max > kMaxBinomRows)
+    if (P.n_max < 1 || P.n_max > kMaxBinomRows)
         return fail(kErrArgs, "relocate: binomial table size must be in [1, 62]");
-    if (num_gaussians == 0) return 0;
-    if (!means3d || !log_scales || !quats || !logit_colors || !logit_opacities)
+    if (P.n == 0) return 0;
+    if (!P.means || !P.log_scales || !P.quats || !P.colors || !P.logit_opac || !P.out_means ||
+        !P.out_log_scales || !P.out_quats || !P.out_colors || !P.out_logit_opac)
         return fail(kErrArgs, "relocate: missing parameter arrays");
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kRelocMaxDevices)
         return fail(kErrRuntime, "relocate: no current device");
     RelocScratch& sc = g_reloc[dev];
     std::lock_guard<std::mutex> lock(sc.mu);
-    int rc = sc.ensure(num_gaussians);
+    int rc = sc.ensure(P.n);
     if (rc) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    RelocParams P;
-    P.means = means3d; P.log_scales = log_scales; P.quats = quats; P.colors = logit_colors;
-    P.logit_opac = logit_opacities;
-    P.n = num_gaussians;
-    P.n_max = n_max;
-    P.min_opacity = min_opacity;
     P.seed_lo = (uint32_t)seed;
     P.seed_hi = (uint32_t)(seed >> 32);
     P.cdf = sc.cdf; P.partials = sc.partials; P.counts = sc.counts; P.src = sc.src;
     P.newv = sc.newv;
-    P.source_out = source;
-    P.reset_out = reset;
-    P.blocks = (num_gaussians + kRelocChunk - 1) / kRelocChunk;
-    const unsigned rows = grid_for(num_gaussians, 256);
-    hipLaunchKernelGGL(reloc_partials_kernel, dim3((unsigned)P.blocks), dim3(256), 0, s, P);
+    P.blocks = (P.n + kRelocChunk - 1) / kRelocChunk;
+    const dim3 chunks((unsigned)P.blocks), rows(grid_for(P.n, 256));
+    hipLaunchKernelGGL(reloc_partials_kernel, chunks, dim3(256), 0, s, P);
     if ((rc = launched("relocate partials"))) return rc;
-    hipLaunchKernelGGL(reloc_scan_partials_kernel, dim3(1), dim3(256), 0, s, P);
+    hipLaunchKernelGGL(reloc_scan_partials_kernel, dim3(1), dim3(kRelocScanThreads), 0, s, P);
     if ((rc = launched("relocate scan"))) return rc;
-    hipLaunchKernelGGL(reloc_cdf_kernel, dim3((unsigned)P.blocks), dim3(256), 0, s, P);
+    hipLaunchKernelGGL(reloc_cdf_kernel, chunks, dim3(256), 0, s, P);
     if ((rc = launched("relocate cdf"))) return rc;
-    hipLaunchKernelGGL(reloc_sample_kernel, dim3(rows), dim3(256), 0, s, P);
+    hipLaunchKernelGGL(reloc_sample_kernel, chunks, dim3(256), 0, s, P);
     if ((rc = launched("relocate sample"))) return rc;
-    hipLaunchKernelGGL(reloc_values_kernel, dim3(rows), dim3(256), 0, s, P);
+    hipLaunchKernelGGL(reloc_values_kernel, chunks, dim3(256), 0, s, P);
     if ((rc = launched("relocate values"))) return rc;
-    hipLaunchKernelGGL(reloc_apply_kernel, dim3(rows), dim3(256), 0, s, P);
+    if (copy)
+        hipLaunchKernelGGL(reloc_apply_kernel<true>, rows, dim3(256), 0, s, P);
+    else
+        hipLaunchKernelGGL(reloc_apply_kernel<false>, rows, dim3(256), 0, s, P);
     return launched("relocate apply");
+}
+
+int splat_mcmc_relocate(splat_stream_t stream, float* means3d, float* log_scales, float* quats,
+                        float* logit_colors, float* logit_opacities, int64_t num_gaussians,
+                        int32_t n_max, float min_opacity, uint64_t seed, int32_t* source,
+                        uint8_t* reset) {
+    RelocParams P{};
+    P.means = P.out_means = means3d;
+    P.log_scales = P.out_log_scales = log_scales;
+    P.quats = P.out_quats = quats;
+    P.colors = P.out_colors = logit_colors;
+    P.logit_opac = P.out_logit_opac = logit_opacities;
+    P.n = num_gaussians; P.n_max = n_max; P.min_opacity = min_opacity;
+    P.source_out = source; P.reset_out = reset;
+    return relocate_impl(stream, P, false, seed);
+}
+
+int splat_mcmc_relocate_copy(splat_stream_t stream, const float* means3d, const float* log_scales,
+                             const float* quats, const float* logit_colors,
+                             const float* logit_opacities, int64_t num_gaussians, int32_t n_max,
+                             float min_opacity, uint64_t seed, float* out_means3d,
+                             float* out_log_scales, float* out_quats, float* out_logit_colors,
+                             float* out_logit_opacities, uint8_t* reset) {
+    RelocParams P{};
+    P.means = means3d; P.log_scales = log_scales; P.quats = quats; P.colors = logit_colors;
+    P.logit_opac = logit_opacities;
+    P.out_means = out_means3d; P.out_log_scales = out_log_scales; P.out_quats = out_quats;
+    P.out_colors = out_logit_colors; P.out_logit_opac = out_logit_opacities;
+    P.n = num_gaussians; P.n_max = n_max; P.min_opacity = min_opacity;
+    P.reset_out = reset;
+    return relocate_impl(stream, P, true, seed);
 }
 
 int splat_mcmc_inject_noise(splat_stream_t stream, const float* means3d, const float* log_scales,

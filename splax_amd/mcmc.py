@@ -62,22 +62,28 @@ def compute_relocation(opacities: torch.Tensor, scales: torch.Tensor, ratios: to
     return new_o, new_s
 
 
+def _check_rows(arrays) -> int:
+    """The gaussian count of the five parameter arrays, each contiguous float32 of one row per
+    gaussian."""
+    n = arrays[0].shape[0]
+    for name, t, w in zip(("means3d", "log_scales", "quats", "logit_colors", "logit_opacities"),
+                          arrays, (3, 3, 4, 3, 1)):
+        if t.dtype != torch.float32 or not t.is_contiguous():
+            raise ValueError(f"{name} must be a contiguous float32 tensor")
+        if t.numel() != n * w:
+            raise ValueError(f"{name} must have {w} values per gaussian, got shape "
+                             f"{tuple(t.shape)} for {n} gaussians")
+    return n
+
+
 def relocate_(key: int, means3d: torch.Tensor, log_scales: torch.Tensor, quats: torch.Tensor,
               logit_colors: torch.Tensor, logit_opacities: torch.Tensor, binoms: torch.Tensor,
               min_opacity: float = 0.005,
               return_source: bool = False):
     """In-place ``relocate`` on contiguous float32 GPU tensors; returns the reset mask (bool, N)
     and, with ``return_source``, the reference's ``source`` index per row (int32, N)."""
-    n = means3d.shape[0]
     arrays = (means3d, log_scales, quats, logit_colors, logit_opacities)
-    widths = (3, 3, 4, 3, 1)
-    for name, t, w in zip(("means3d", "log_scales", "quats", "logit_colors", "logit_opacities"),
-                          arrays, widths):
-        if t.dtype != torch.float32 or not t.is_contiguous():
-            raise ValueError(f"{name} must be a contiguous float32 tensor")
-        if t.numel() != n * w:
-            raise ValueError(f"{name} must have {w} values per gaussian, got shape "
-                             f"{tuple(t.shape)} for {n} gaussians")
+    n = _check_rows(arrays)
     dev = _lib.require_gpu(*arrays)
     reset = torch.empty((n,), device=dev, dtype=torch.bool)
     source = torch.empty((n,), device=dev, dtype=torch.int32) if return_source else None
@@ -97,9 +103,21 @@ def relocate(key: int, means3d: torch.Tensor, log_scales: torch.Tensor, quats: t
     Returns the new (means3d, log_scales, quats, logit_colors, logit_opacities), each of the
     input's shape, and the bool mask of rows whose optimizer moments should be zeroed.
     """
-    new = tuple(_f32c(t, "parameter").clone() for t in (means3d, log_scales, quats,
-                                                         logit_colors, logit_opacities))
-    reset = relocate_(key, *new, binoms, min_opacity)
+    arrays = tuple(_f32c(t, "parameter") for t in (means3d, log_scales, quats, logit_colors,
+                                                   logit_opacities))
+    if torch.is_grad_enabled() and any(t.requires_grad for t in arrays):
+        new = tuple(t.clone() for t in arrays)  # copies that keep their inputs' graph
+        return new, relocate_(key, *new, binoms, min_opacity)
+    n = _check_rows(arrays)
+    dev = _lib.require_gpu(*arrays)
+    new = tuple(torch.empty_like(t) for t in arrays)
+    reset = torch.empty((n,), device=dev, dtype=torch.bool)
+    with torch.cuda.device(dev):
+        st = _lib.lib().splat_mcmc_relocate_copy(
+            _lib.stream_handle(dev), *(_lib.ptr(t) for t in arrays), n, _n_max(binoms),
+            float(min_opacity), int(key) & 0xFFFFFFFFFFFFFFFF, *(_lib.ptr(t) for t in new),
+            _lib.ptr(reset))
+    _lib.check(st, "relocate")
     return new, reset
 
 

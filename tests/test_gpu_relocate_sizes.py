@@ -1,0 +1,50 @@
+"""Relocation at the sizes where its scans, its sixteen-way search and its compaction can go wrong
+(one row, the edges of a search round and of a 1024-row chunk, several chunks) and at no, few, most
+and all rows dead: sources and copied parameters bit for bit the oracle's, relocated values within
+one float32 ulp (double pow / log of two math libraries), and relocate() bit for bit relocate_()."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import train_oracle as TO
+from splax_amd import mcmc
+
+pytestmark = pytest.mark.gpu
+
+
+def _ulps(a, b):
+    return np.abs(a.view(np.int32).astype(np.int64) - b.view(np.int32).astype(np.int64))
+
+
+@pytest.mark.parametrize("n,dead", [
+    *((n, d) for n in (1, 2, 15, 16, 17, 257, 1023, 1024, 1025, 5000)
+      for d in (0.0, 0.05, 0.9, 1.0)),
+    (4096 * 1024, 0.002),  # the most chunk prefixes that are searched in LDS
+    (4096 * 1024 + 1, 0.002),
+])
+def test_relocate_sizes(n, dead):
+    rng = np.random.default_rng(1000 * n + int(100 * dead))
+    f32 = lambda *s: rng.normal(size=s).astype(np.float32)  # noqa: E731
+    p = [f32(n, 3), f32(n, 3) - 4, f32(n, 4), f32(n, 3), f32(n, 1)]
+    is_dead = rng.uniform(size=(n, 1)) < dead
+    p[4] = np.where(is_dead, np.float32(-9), p[4]).astype(np.float32)
+    dev = [torch.from_numpy(a).cuda() for a in p]
+    binoms = mcmc.make_binoms(51)
+    inplace = [t.clone() for t in dev]
+    reset, source = mcmc.relocate_(7, *inplace, binoms, return_source=True)
+    new, reset2 = mcmc.relocate(7, *dev, binoms)
+    assert all(torch.equal(a, torch.from_numpy(b).cuda()) for a, b in zip(dev, p))
+    assert torch.equal(reset, reset2)
+    assert all(torch.equal(a, b) for a, b in zip(new, inplace))
+    *ref, ref_source, ref_reset = TO.relocate(7, *p, n_max=51, min_opacity=0.005)
+    assert np.array_equal(source.cpu().numpy(), ref_source)
+    assert np.array_equal(reset.cpu().numpy(), np.asarray(ref_reset).astype(bool))
+    for k, (got, want) in enumerate(zip(new, ref)):
+        got, want = got.cpu().numpy(), np.asarray(want, np.float32).reshape(p[k].shape)
+        if k in (1, 4):
+            assert int(_ulps(got, want).max()) <= 1, k
+        else:
+            assert np.array_equal(got, want), k
