@@ -229,6 +229,12 @@ int splat_sort_and_bin(splat_stream_t stream, const float* xys, const float* dep
                        int64_t* sorted_keys, int32_t* sorted_ids, int64_t capacity,
                        int32_t* tile_bins, int64_t* num_intersects);
 
+/* Replaces splax.transform_ids (splax/_project/_project.py:120-136): transform_ids [n] int32 = the
+ * index of the slice that holds each gaussian, -1 outside them. slices: num_slices (start, stop)
+ * pairs in HOST memory, disjoint and inside [0, n). */
+int splat_transform_ids(splat_stream_t stream, const int32_t* slices, int32_t num_slices,
+                        int64_t num_gaussians, int32_t* transform_ids);
+
 /* Replaces the _use_32bit_keys switch (splax/_rasterize/_sort/_sort.py:23-26), which the
  * reference's tests patch: force != 0 makes every sort take the 64-bit key (process-wide). */
 int splat_set_wide_keys(int force);

@@ -61,6 +61,19 @@ def project_fwd(means, scales, quats, viewmat, opac, transforms, transform_ids, 
     return xys, depths, radii, conics, nth, cum
 
 
+def transform_ids(n, slices, dev):
+    """The (n,) int32 slice indices of n gaussians on a GPU, for checked disjoint slices."""
+    _lib.require_gpu()
+    ids = torch.empty((n,), device=dev, dtype=torch.int32)
+    flat = [int(v) for pair in slices for v in pair]
+    with torch.cuda.device(ids.device):
+        st = _lib.lib().splat_transform_ids(
+            _lib.stream_handle(ids.device), (ctypes.c_int32 * len(flat))(*flat), len(flat) // 2, n,
+            ids.data_ptr())
+    _lib.check(st, "transform_ids")
+    return ids
+
+
 def project_bwd(means, scales, quats, viewmat, radii, conics, v_xy, v_depth, v_conic,
                 transforms, transform_ids, *, n, B, num_transforms, has_transforms, f,
                 glob_scale, quats_wxyz=False, fold=False, want_viewmat=True):

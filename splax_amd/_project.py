@@ -201,6 +201,9 @@ def transform_ids(n: int, slices: Sequence[tuple[int, int]],
     for (_, prev_stop), (start, _) in zip(ordered, ordered[1:]):
         if start < prev_stop:
             raise ValueError(f"gaussian slices overlap: {list(slices)}")
+    dev = torch.device("cpu" if device is None else device)
+    if dev.type == "cuda":
+        return _ops.transform_ids(n, slices, dev)
     ids = torch.full((n,), -1, dtype=torch.int32, device=device)
     for k, (start, stop) in enumerate(slices):
         ids[start:stop] = k

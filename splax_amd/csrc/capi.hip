@@ -672,6 +672,23 @@ int splat_project_bwd(splat_stream_t stream, const float* means3d, int64_t rows_
     return rc;
 }
 
+int splat_transform_ids(splat_stream_t stream, const int32_t* slices, int32_t num_slices,
+                        int64_t num_gaussians, int32_t* transform_ids) {
+    if (num_slices < 0 || num_gaussians < 0 || num_gaussians >= ((int64_t)1 << 31) ||
+        (num_slices > 0 && !slices))
+        return fail(kErrArgs, "transform_ids: invalid sizes");
+    for (int32_t k = 0; k < num_slices; ++k)
+        if (slices[2 * k] < 0 || slices[2 * k] >= slices[2 * k + 1] ||
+            slices[2 * k + 1] > num_gaussians)
+            return fail(kErrArgs, "transform_ids: slice outside [0, num_gaussians)");
+    if (num_gaussians == 0) return 0;
+    if (!transform_ids) return fail(kErrArgs, "transform_ids: missing output buffer");
+    if (launch_transform_ids(slices, num_slices, num_gaussians, transform_ids,
+                             static_cast<hipStream_t>(stream)))
+        return fail(kErrLaunch, "transform_ids launch failed");
+    return 0;
+}
+
 // blend: the call blends (colours, opacities and background are read), not only sorts.
 static int check_raster(const RasterInputs& in, int32_t B_out, bool blend = true) {
     if (in.n <= 0 || in.B_geom <= 0 || in.img_h <= 0 || in.img_w <= 0)

@@ -13,9 +13,9 @@
 // project_bwd: one thread per flat item, restating _project_bwd_kernel
 // (splax/_project/_kernels.py:356-484); the per-image viewmat gradient (formed only when asked
 // for) is reduced per wave with DPP, then per workgroup in LDS into 12 partials per (image,
-// workgroup), which viewmat_reduce_kernel sums in a fixed order. The transform gradient follows
-// the reference's three cases: a workgroup whose gaussians share one transform reduces in LDS
-// and adds with one atomic per entry, a workgroup on a slice boundary adds per thread.
+// workgroup), which viewmat_reduce_kernel sums in a fixed order. The transform gradient: a
+// workgroup whose gaussians share one transform reduces in LDS and adds with one atomic per
+// entry, a mixed one per wave and transform.
 #include "splat_common.hpp"
 #include "splat_internal.hpp"
 
@@ -705,23 +705,24 @@ __global__ void __launch_bounds__(kProjThreads) project_bwd_kernel(ProjectBwdPar
             P.view_partials[((int64_t)image_id * P.blocks_per_image + local_block) * 12 + tid] = v;
         }
     }
-    // Transform gradient: uniform block -> block reduction; mixed -> per-thread atomics
-    // (splax/_project/_kernels.py:461-484).
+    // Transform gradient (splax/_project/_kernels.py:461-484): a workgroup of one transform adds
+    // its sums with one atomic per entry; in a mixed one (a slice boundary, or ids in any order)
+    // each wave sums the lanes of one transform at a time and adds those. Twelve atomics per
+    // thread into the same twelve words there kept this kernel at 87 us for 150K gaussians in
+    // twelve slices, 13 us so.
     if (kTf) {
-        int32_t id = in_range ? tf_id : -1;
-        int32_t tmin = block_min_i32(in_range ? tf_id : 2147483647, s_tf);
-        int32_t tmax = block_max_i32(in_range ? tf_id : (-2147483647 - 1), s_tf);
-        (void)id;
+        const int32_t tmin = block_min_i32(in_range ? tf_id : 2147483647, s_tf);
+        const int32_t tmax = block_max_i32(in_range ? tf_id : (-2147483647 - 1), s_tf);
+        float rt[12];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+#pragma unroll
+            for (int b = 0; b < 3; ++b) rt[4 * a + b] = vRtf[3 * a + b];
+            rt[4 * a + 3] = vttf[a];
+        }
         // ids at or beyond num_transforms are static (apply_transform), like negative ones
         if (tmin == tmax && tmin >= 0 && tmin < P.num_transforms) {
             __syncthreads();
-            float rt[12];
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-#pragma unroll
-                for (int b = 0; b < 3; ++b) rt[4 * a + b] = vRtf[3 * a + b];
-                rt[4 * a + 3] = vttf[a];
-            }
 #pragma unroll
             for (int k = 0; k < 12; ++k) {
                 float v = wave_sum_to_lane63(rt[k]);
@@ -733,14 +734,21 @@ __global__ void __launch_bounds__(kProjThreads) project_bwd_kernel(ProjectBwdPar
                 int64_t slot = (int64_t)image_id * P.num_transforms + tmin;
                 atomicAdd(P.v_transforms + slot * 16 + tid, v);
             }
-        } else if (moved && tmin != tmax) {
-            int64_t slot = (int64_t)image_id * P.num_transforms + tf_id;
-            float* dst = P.v_transforms + slot * 16;
+        } else if (tmin != tmax) {
+            // every lane is active; only the lanes of moved gaussians hold sums
+            uint64_t todo = __builtin_amdgcn_ballot_w64(moved);
+            while (todo != 0ull) {
+                const int32_t cur = __builtin_amdgcn_readlane(tf_id, __builtin_ctzll(todo));
+                const bool mine = moved && tf_id == cur;
+                float sum = 0.0f;
 #pragma unroll
-            for (int a = 0; a < 3; ++a) {
-#pragma unroll
-                for (int b = 0; b < 3; ++b) atomicAdd(dst + 4 * a + b, vRtf[3 * a + b]);
-                atomicAdd(dst + 4 * a + 3, vttf[a]);
+                for (int k = 0; k < 12; ++k) {
+                    const float v = lane63(wave_sum_to_lane63(mine ? rt[k] : 0.0f));
+                    sum = lane == k ? v : sum;
+                }
+                const int64_t slot = (int64_t)image_id * P.num_transforms + cur;
+                if (lane < 12) atomicAdd(P.v_transforms + slot * 16 + lane, sum);
+                todo &= ~__builtin_amdgcn_ballot_w64(mine);
             }
         }
     }
@@ -757,6 +765,44 @@ __global__ void __launch_bounds__(kProjThreads) project_bwd_kernel(ProjectBwdPar
             P.wxyz ? make_float4(fq[3], fq[0], fq[1], fq[2])
                    : make_float4(fq[0], fq[1], fq[2], fq[3]);
     }
+}
+
+// transform_ids (splax/_project/_project.py:120-136): the slice each gaussian lies in, -1 for none.
+// The slices come as kernel arguments, kIdSlices to a launch (one launch for all gaussians, where a
+// fill per slice took 2 us of GPU and 5 us of host time each); launches after the first write
+// only the gaussians of their slices.
+constexpr int kIdSlices = 64;
+struct TransformIdParams {
+    int32_t start[kIdSlices], stop[kIdSlices];
+    int32_t count, first_id;
+    int64_t n;
+    int32_t* ids;
+};
+__global__ void __launch_bounds__(256) transform_ids_kernel(TransformIdParams P) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= P.n) return;
+    int32_t id = -1;
+    for (int k = 0; k < P.count; ++k)
+        id = i >= P.start[k] && i < P.stop[k] ? P.first_id + k : id;
+    if (P.first_id == 0 || id >= 0) P.ids[i] = id;
+}
+
+int launch_transform_ids(const int32_t* slices, int32_t count, int64_t n, int32_t* ids,
+                         hipStream_t stream) {
+    for (int32_t k0 = 0; k0 == 0 || k0 < count; k0 += kIdSlices) {
+        TransformIdParams P{};
+        P.count = count - k0 < kIdSlices ? count - k0 : kIdSlices;
+        P.first_id = k0;
+        for (int32_t k = 0; k < P.count; ++k) {
+            P.start[k] = slices[2 * (k0 + k)];
+            P.stop[k] = slices[2 * (k0 + k) + 1];
+        }
+        P.n = n;
+        P.ids = ids;
+        hipLaunchKernelGGL(transform_ids_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+                           stream, P);
+    }
+    return hipGetLastError() == hipSuccess ? 0 : kErrLaunch;
 }
 
 // One workgroup per image: the image's workgroup partials summed in a fixed order (each thread a

@@ -62,6 +62,10 @@ struct ProjectBwdArgs {
     int32_t fold = 0;        // v_mean3d / v_scale / v_quat summed over the images (n rows)
 };
 
+// ids[i] of n gaussians from `count` host (start, stop) pairs.
+int launch_transform_ids(const int32_t* slices, int32_t count, int64_t n, int32_t* ids,
+                         hipStream_t stream);
+
 // Geometry of one sort_and_bin call (splax/_rasterize/_sort/_sort.py:51-60).
 // packed: the 32-bit key (at least 16 depth bits left); otherwise the 64-bit key, which
 // overflows when image + tile bits exceed 32 (splax/_rasterize/_sort/_sort.py:56-66).
