@@ -29,6 +29,9 @@ def batch_shape(named: dict[str, tuple[torch.Tensor | None, int]]) -> tuple[int,
         if t.ndim < base:
             raise ValueError(f"{name}: expected at least {base} dims, got {tuple(t.shape)}")
         leads.append((name, tuple(t.shape[: t.ndim - base])))
+    batched = {lead for _, lead in leads if lead}
+    if len(batched) < 2:  # nothing batched, or one batch shape: no broadcasting
+        return batched.pop() if batched else ()
     try:
         return tuple(torch.broadcast_shapes(*(lead for _, lead in leads)))
     except RuntimeError as e:

@@ -131,21 +131,44 @@ def check(status: int, what: str) -> None:
 
 def require_gpu(*tensors: torch.Tensor) -> torch.device:
     """All tensors must live on one ROCm device; returns it."""
-    if not torch.cuda.is_available():
-        raise RuntimeError("splax_amd needs a ROCm GPU (torch.cuda.is_available() is False)")
     dev = None
     for t in tensors:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
+            if not torch.cuda.is_available():
+                break
             raise ValueError(f"expected a GPU tensor, got one on {t.device}")
         if dev is None:
             dev = t.device
         elif t.device != dev:
             raise ValueError(f"tensors on different devices: {dev} and {t.device}")
-    if dev is None:
-        dev = torch.device("cuda", torch.cuda.current_device())
-    return dev
+    else:
+        if dev is not None:
+            return dev
+    if not torch.cuda.is_available():
+        raise RuntimeError("splax_amd needs a ROCm GPU (torch.cuda.is_available() is False)")
+    return torch.device("cuda", torch.cuda.current_device())
+
+
+class _Here:
+    """The device guard of a call whose device is the current one already."""
+
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_HERE = _Here()
+
+
+def on_device(device: torch.device):
+    """``torch.cuda.device(device)``, without its two device switches where it is current."""
+    if torch.cuda.current_device() == device.index:
+        return _HERE
+    return torch.cuda.device(device)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
@@ -153,7 +176,8 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 
 def stream_handle(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(
+        torch.cuda.current_device() if device.index is None else device.index)
 
 
 def set_stage_timing(stages=None) -> None:

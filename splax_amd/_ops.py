@@ -8,6 +8,7 @@ operands' device and enqueues the library call on torch's current stream of that
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import NamedTuple, Optional
 
 import torch
@@ -50,7 +51,7 @@ def project_fwd(means, scales, quats, viewmat, opac, transforms, transform_ids, 
     if total == 0:
         return xys, depths, radii, conics, nth, cum
     p = _lib.ptr
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().splat_project_fwd(
             _lib.stream_handle(dev), p(means), rows(means, 3), p(scales), rows(scales, 3),
             p(quats), rows(quats, 4), p(viewmat), rows(viewmat, 4), p(opac), opac.numel(),
@@ -66,7 +67,7 @@ def transform_ids(n, slices, dev):
     _lib.require_gpu()
     ids = torch.empty((n,), device=dev, dtype=torch.int32)
     flat = [int(v) for pair in slices for v in pair]
-    with torch.cuda.device(ids.device):
+    with _lib.on_device(ids.device):
         st = _lib.lib().splat_transform_ids(
             _lib.stream_handle(ids.device), (ctypes.c_int32 * len(flat))(*flat), len(flat) // 2, n,
             ids.data_ptr())
@@ -98,7 +99,7 @@ def project_bwd(means, scales, quats, viewmat, radii, conics, v_xy, v_depth, v_c
     if has_transforms:
         v_tf = torch.empty((B * num_transforms, 4, 4), device=dev, dtype=torch.float32)
     p = _lib.ptr
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().splat_project_bwd(
             _lib.stream_handle(dev), p(means), rows(means, 3), p(scales), rows(scales, 3),
             p(quats), rows(quats, 4), p(viewmat), rows(viewmat, 4), p(radii), radii.numel(),
@@ -129,7 +130,7 @@ def rasterize_fwd(colors, opac, map_opac, background, xys, depths, radii, conics
     args = (_lib.stream_handle(dev), p(colors), rows(colors, 3), p(opac), opac.numel(),
             p(map_opac), map_opac.numel(), p(background), rows(background, 3), p(xys), p(depths),
             p(radii), p(conics), p(cum), n, B, H, W, p(Ts), p(fidx), p(img))
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         if render_depth:
             st = _lib.lib().splat_rasterize_depth_fwd(*args, p(depth), ctypes.byref(m))
         else:
@@ -206,7 +207,7 @@ def rasterize_fwd_keep(colors, opac, map_opac, background, xys, depths, radii, c
     for _ in range(2):
         ids = torch.empty((max(cap, 1),), device=dev, dtype=torch.int32)
         pos = torch.empty((max(cap, 1),), device=dev, dtype=torch.int32)
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             st = _lib.lib().splat_rasterize_fwd_keep(
                 _lib.stream_handle(dev), p(colors), rows(colors, 3), p(opac), opac.numel(),
                 p(map_opac), map_opac.numel(), p(background), rows(background, 3), p(xys),
@@ -225,15 +226,78 @@ def rasterize_fwd_keep(colors, opac, map_opac, background, xys, depths, radii, c
     return img, Ts, fidx, KeptSort(ids, pos, bins, M, recs, order), depth
 
 
-class RenderKept(NamedTuple):
+class RenderKept:
     """What splat_render_fwd keeps for splat_render_bwd: the projection outputs and the
-    rasterizer's kept lists."""
-    xys: torch.Tensor
-    depths: torch.Tensor
-    radii: torch.Tensor
-    conics: torch.Tensor
-    cum: torch.Tensor
-    sort: KeptSort
+    rasterizer's kept lists, in two buffers (one allocation each where eleven small ones took
+    longer on the host than a small render's kernels). ``work`` (float32) holds the arrays of
+    ``_FIELDS``, ``lists`` (int32) the ``capacity`` sorted ids and, when a backward may follow,
+    as many emission positions; ``M`` is the intersection count."""
+
+    __slots__ = ("work", "lists", "items", "bins_rows", "M", "capacity", "with_pos")
+    # name -> (words per item, words per (image, tile), dtype, row width)
+    _FIELDS = {"xys": (2, 0, torch.float32, 2), "depths": (1, 0, torch.float32, 0),
+               "conics": (3, 0, torch.float32, 3), "radii": (1, 0, torch.int32, 0),
+               "nth": (1, 0, torch.int32, 0), "cum": (1, 0, torch.int32, 0),
+               "records": (16, 0, torch.float32, 16), "bins": (0, 2, torch.int32, 2),
+               "order": (0, 1, torch.int32, 0)}
+
+    def __init__(self, items, bins_rows, with_pos, work=None, lists=None, M=0, capacity=0,
+                 device=None):
+        self.items, self.bins_rows, self.with_pos = items, bins_rows, with_pos
+        self.lists, self.M, self.capacity = lists, M, capacity
+        words = self._layout(items, bins_rows)[1]
+        if work is None:
+            work = torch.empty((words,), device=device, dtype=torch.float32)
+        elif (work.numel() != words or work.dtype != torch.float32 or not work.is_contiguous()
+              or lists.dtype != torch.int32 or not lists.is_contiguous()
+              or lists.numel() < (2 if with_pos else 1) * capacity):
+            raise ValueError("the kept buffers are not those of a forward of these sizes")
+        self.work = work
+
+    @staticmethod
+    @functools.lru_cache(maxsize=64)
+    def _layout(items, bins_rows):
+        """Word offset of every array (256-byte steps) and the words in all."""
+        at, offsets = 0, {}
+        for name, (per_item, per_tile, _, _) in RenderKept._FIELDS.items():
+            offsets[name] = at
+            at += (per_item * items + per_tile * bins_rows + 63) // 64 * 64
+        return offsets, at
+
+    def allocate_lists(self, capacity):
+        self.capacity = capacity
+        words = (max(capacity, 1) + 63) // 64 * 64
+        self.lists = torch.empty((words * (2 if self.with_pos else 1),),
+                                 device=self.work.device, dtype=torch.int32)
+
+    def pointers(self):
+        """name -> address, with ids and pos (None without a backward)."""
+        base = self.work.data_ptr()
+        out = {k: base + 4 * v for k, v in self._layout(self.items, self.bins_rows)[0].items()}
+        out["ids"] = self.lists.data_ptr()
+        out["pos"] = out["ids"] + 2 * self.lists.numel() if self.with_pos else None
+        return out
+
+    def _array(self, name):
+        per_item, per_tile, dtype, width = self._FIELDS[name]
+        rows = self.items if per_item else self.bins_rows
+        at = self._layout(self.items, self.bins_rows)[0][name]
+        t = self.work[at:at + (per_item + per_tile) * rows].view(dtype)
+        return t.view(rows, width) if width else t
+
+    xys = property(lambda self: self._array("xys"))
+    depths = property(lambda self: self._array("depths"))
+    radii = property(lambda self: self._array("radii"))
+    conics = property(lambda self: self._array("conics"))
+    cum = property(lambda self: self._array("cum"))
+
+    @property
+    def sort(self) -> KeptSort:
+        half = self.lists.numel() // (2 if self.with_pos else 1)
+        n = max(self.capacity, 1)
+        return KeptSort(self.lists[:n], self.lists[half:half + n] if self.with_pos else None,
+                        self._array("bins"), self.M, self._array("records"),
+                        self._array("order"))
 
 
 def render_fwd(means, scales, quats_wxyz, colors, opac, viewmat, background, transforms,
@@ -257,40 +321,38 @@ def render_fwd(means, scales, quats_wxyz, colors, opac, viewmat, background, tra
         loss_target = _f32(loss_target)
     tiles = ((W + 15) // 16) * ((H + 15) // 16)
     e = lambda *shape, dt=torch.float32: torch.empty(shape, device=dev, dtype=dt)  # noqa: E731
-    xys, depths, conics = e(total, 2), e(total), e(total, 3)
-    radii, nth, cum = e(total, dt=torch.int32), e(total, dt=torch.int32), e(total, dt=torch.int32)
     img = e(B * H, W, 3)
     Ts, fidx = (e(B * H, W), e(B * H, W, dt=torch.int32)) if backward else (None, None)
     depth = e(B * H, W) if render_depth else None
-    bins, recs, order = e(B * tiles, 2, dt=torch.int32), e(total, 16), e(B * tiles, dt=torch.int32)
+    kept = RenderKept(total, B * tiles, backward, device=dev)
     key = str(dev)
     cap = _keep_capacity(key, (B, n, tiles))
     m = ctypes.c_int64(0)
     p = _lib.ptr
-    for _ in range(2):
-        ids = e(max(cap, 1), dt=torch.int32)
-        pos = e(max(cap, 1), dt=torch.int32) if backward else None
-        with torch.cuda.device(dev):
+    with _lib.on_device(dev):
+        for _ in range(2):
+            kept.allocate_lists(cap)
+            k = kept.pointers()
             st = _lib.lib().splat_render_fwd(
                 _lib.stream_handle(dev), p(means), rows(means, 3), p(scales), rows(scales, 3),
                 p(quats_wxyz), rows(quats_wxyz, 4), p(viewmat), rows(viewmat, 4), p(opac),
                 opac.numel(), p(colors), rows(colors, 3), p(background), rows(background, 3),
                 p(transforms), rows(transforms, 16), p(transform_ids), n, num_transforms,
                 int(has_transforms), B, H, W, f[0], f[1], c[0], c[1], glob_scale, clip_thresh, 1,
-                int(compensate), p(xys), p(depths), p(radii), p(conics), p(nth), p(cum), cap,
-                p(ids), p(pos), p(bins), p(recs), p(order), p(Ts), p(fidx), p(img), p(depth),
-                ctypes.byref(m), p(loss_target) if loss_kind else None, int(loss_kind),
+                int(compensate), k["xys"], k["depths"], k["radii"], k["conics"], k["nth"],
+                k["cum"], cap, k["ids"], k["pos"], k["bins"], k["records"], k["order"], p(Ts),
+                p(fidx), p(img), p(depth), ctypes.byref(m),
+                p(loss_target) if loss_kind else None, int(loss_kind),
                 p(loss_out) if loss_kind else None)
-        if st == _lib.ERR_TOO_MANY and m.value > cap:
-            cap = int(m.value * 1.25) + 1
-            _KEEP_CAPACITY[key] = cap
-            continue
-        break
+            if st == _lib.ERR_TOO_MANY and m.value > cap:
+                cap = int(m.value * 1.25) + 1
+                _KEEP_CAPACITY[key] = cap
+                continue
+            break
     _lib.check(st, "render")
-    M = int(m.value)
-    if M > _KEEP_CAPACITY.get(key, 0):
-        _KEEP_CAPACITY[key] = int(M * 1.25) + 1
-    kept = RenderKept(xys, depths, radii, conics, cum, KeptSort(ids, pos, bins, M, recs, order))
+    kept.M = int(m.value)
+    if kept.M > _KEEP_CAPACITY.get(key, 0):
+        _KEEP_CAPACITY[key] = int(kept.M * 1.25) + 1
     return img, Ts, fidx, kept, depth
 
 
@@ -324,17 +386,17 @@ def render_bwd(means, scales, quats_wxyz, colors, opac, viewmat, background, tra
     v_colors, v_opac = e(rows_out, 3), e(rows_out)
     v_view = e(B * 4, 4) if want_viewmat else None
     v_tf = e(B * num_transforms, 4, 4) if has_transforms else None
-    ks = kept.sort
+    k = kept.pointers()
     p = _lib.ptr
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().splat_render_bwd(
             _lib.stream_handle(dev), p(means), rows(means, 3), p(scales), rows(scales, 3),
             p(quats_wxyz), rows(quats_wxyz, 4), p(viewmat), rows(viewmat, 4), p(opac),
             opac.numel(), p(colors), rows(colors, 3), p(background), rows(background, 3),
             p(transforms), rows(transforms, 16), p(_i32(transform_ids)), n, num_transforms,
             int(has_transforms), B, H, W, f[0], f[1], glob_scale, 1, int(compensate),
-            p(kept.xys), p(kept.depths), p(kept.radii), p(kept.conics), p(kept.cum), p(ks.ids),
-            p(ks.pos), p(ks.bins), p(ks.records), p(ks.order), ks.M, p(final_Ts), p(final_idx),
+            k["xys"], k["depths"], k["radii"], k["conics"], k["cum"], k["ids"], k["pos"],
+            k["bins"], k["records"], k["order"], kept.M, p(final_Ts), p(final_idx),
             p(v_out), 0 if v_out is None else v_out.numel() // (3 * W), p(vd),
             0 if vd is None else vd.numel() // W, p(v_means), p(v_scales), p(v_quats),
             p(v_colors), p(v_opac), p(v_view), p(v_tf), int(fold),
@@ -386,7 +448,7 @@ def rasterize_bwd_sorted(colors, opac, background, xys, depths, conics, cum, kep
     if fold:  # shared colours and opacities: the library sums their per-image rows
         v_colors, v_opac = v_colors[:n], v_opac[:n]
     p = _lib.ptr
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().splat_rasterize_bwd_sorted(
             _lib.stream_handle(dev), p(colors), rows(colors, 3), p(opac), opac.numel(),
             p(background), rows(background, 3), p(xys), p(depths), p(conics), p(cum), p(ids),
@@ -416,7 +478,7 @@ def rasterize_bwd(colors, opac, map_opac, background, xys, depths, radii, conics
             p(map_opac), map_opac.numel(), p(background), rows(background, 3), p(xys), p(depths),
             p(radii), p(conics), p(cum), p(final_Ts), p(final_idx), p(v_out),
             v_out.numel() // (3 * W))
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         if vd is None:
             st = _lib.lib().splat_rasterize_bwd(*args, n, B_out, B_geom, H, W, p(v_colors),
                                                 p(v_opac), p(v_xy), p(v_conic))
@@ -445,7 +507,7 @@ def sort_and_bin(xys, depths, radii, conics, map_opac, cum, *, n, B, img_shape, 
     bins = torch.empty((B * tiles, 2), device=dev, dtype=torch.int32)
     m = torch.zeros(1, dtype=torch.int64)
     p = _lib.ptr
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().splat_sort_and_bin(
             _lib.stream_handle(dev), p(xys), p(depths), p(radii), p(conics), p(map_opac),
             map_opac.numel(), p(cum), n, B, H, W, p(keys), p(ids), capacity, p(bins),

@@ -76,12 +76,12 @@ class _ProjectFn(torch.autograd.Function):
         g_quats = fold(v_quat, quats, 4) if ctx.needs_input_grad[2] else None
         g_view = None
         if ctx.needs_input_grad[3]:
-            g_view = v_view.reshape(B, 4, 4)
-            g_view = g_view.reshape(viewmat.shape) if viewmat.ndim == 3 else g_view.sum(0)
+            g_view = v_view.reshape(viewmat.shape) if viewmat.ndim == 3 or B == 1 else \
+                v_view.reshape(B, 4, 4).sum(0)
         g_tf = None
         if has_tf and ctx.needs_input_grad[5]:
-            g_tf = v_tf.reshape(B, K, 4, 4)
-            g_tf = g_tf.reshape(transforms.shape) if transforms.ndim == 4 else g_tf.sum(0)
+            g_tf = v_tf.reshape(transforms.shape) if transforms.ndim == 4 or B == 1 else \
+                v_tf.reshape(B, K, 4, 4).sum(0)
         return g_means, g_scales, g_quats, g_view, None, g_tf, None, None
 
 
@@ -91,11 +91,10 @@ _NO_TF: dict = {}
 def _no_transforms(dev: torch.device):
     """The reference's dummy (1, 4, 4) transforms and (1,) ids of -1 (splax/_project/_project.py:71-73),
     made once per device."""
-    key = str(dev)
-    if key not in _NO_TF:
-        _NO_TF[key] = (torch.zeros((1, 4, 4), device=dev, dtype=torch.float32),
+    if dev not in _NO_TF:
+        _NO_TF[dev] = (torch.zeros((1, 4, 4), device=dev, dtype=torch.float32),
                        torch.full((1,), -1, device=dev, dtype=torch.int32))
-    return _NO_TF[key]
+    return _NO_TF[dev]
 
 
 def project(mean3ds: torch.Tensor, scales: torch.Tensor, quats: torch.Tensor,

@@ -9,6 +9,7 @@ and conics, and on the depth path also depths.
 
 from __future__ import annotations
 
+import functools
 import math
 
 import torch
@@ -32,6 +33,7 @@ def key_layout(B: int, H: int, W: int) -> dict:
             "overflow": not packed and image_bits + tile_bits > 32}
 
 
+@functools.lru_cache(maxsize=64)
 def check_key_fits(B: int, H: int, W: int) -> None:
     """Raise like the reference when even the 64-bit key cannot hold the image and tile ids
     (splax/_rasterize/_sort/_sort.py:61-66)."""

@@ -19,6 +19,11 @@ from splax_amd._project import _no_transforms, transform_ids
 from splax_amd._rasterize import check_key_fits
 
 
+def _shaped(t: torch.Tensor, shape) -> torch.Tensor:
+    """t.reshape(shape), t itself (no view, no autograd node) where it has that shape."""
+    return t if t.shape == tuple(shape) else t.reshape(shape)
+
+
 class _LogParamsFn(torch.autograd.Function):
     """exp(log_scales), quats / (|quats| + 1e-8), sigmoid(logit_colors), sigmoid(logit_opac)
     (splax/_render.py:161-164) over flat rows."""
@@ -35,7 +40,7 @@ class _LogParamsFn(torch.autograd.Function):
         dev = _lib.require_gpu(*ins)
         outs = [torch.empty_like(t) for t in ins]
         p = _lib.ptr
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             st = _lib.lib().splat_log_params_fwd(_lib.stream_handle(dev), *map(p, ins), n,
                                                  *map(p, outs))
         _lib.check(st, "log_params_fwd")
@@ -52,7 +57,7 @@ class _LogParamsFn(torch.autograd.Function):
         outs = [torch.empty_like(t) for t in ins]
         dev = ins[0].device
         p = _lib.ptr
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             st = _lib.lib().splat_log_params_bwd(_lib.stream_handle(dev), *map(p, ins), n,
                                                  *map(p, vs), *map(p, outs))
         _lib.check(st, "log_params_bwd")
@@ -77,20 +82,18 @@ def _fused_forward(means, scales, quats, colors, opac, viewmat, background, tran
 
 
 def _save_forward(ctx, operands, Ts, fidx, kept, statics, extra=()):
-    ks = kept.sort
-    ctx.save_for_backward(*operands, Ts, fidx, kept.xys, kept.depths, kept.radii, kept.conics,
-                          kept.cum, ks.ids, ks.pos, ks.bins, ks.records, ks.order, *extra)
+    ctx.save_for_backward(*operands, Ts, fidx, kept.work, kept.lists, *extra)
     ctx.statics = statics
-    ctx.num_intersects = ks.M
+    ctx.kept = (kept.items, kept.bins_rows, kept.M, kept.capacity)
     ctx.set_materialize_grads(False)
 
 
-def _backward(ctx, v_img, v_depth, loss=None):
-    """splat_render_bwd for a forward saved by _save_forward; loss: (kind, target, image,
-    v_loss) when the forward fused the loss (v_img then unused). Returns the cotangents of
-    means, scales, quats, colors, opacities, viewmat and transforms."""
-    (means, scales, quats, colors, opac, viewmat, background, transforms, tf_ids, Ts, fidx,
-     xys, depths, radii, conics, cum, ids, pos, bins, recs, order) = ctx.saved_tensors[:21]
+def _backward(ctx, saved, v_img, v_depth, loss=None):
+    """splat_render_bwd for a forward saved by _save_forward (saved: its saved tensors); loss:
+    (kind, target, image, v_loss) when the forward fused the loss (v_img then unused). Returns
+    the cotangents of means, scales, quats, colors, opacities, viewmat and transforms."""
+    (means, scales, quats, colors, opac, viewmat, background, transforms, tf_ids, Ts, fidx, work,
+     lists) = saved[:13]
     n, B, K, has_tf, img_shape, f, c, glob_scale, clip_thresh, compensate, render_depth = \
         ctx.statics
     H, W = img_shape
@@ -102,8 +105,8 @@ def _backward(ctx, v_img, v_depth, loss=None):
                                               (colors, 3), (opac, 1))]
     fold_here = B > 1 and all(shared)
     flat = lambda t, w: t.reshape(-1, w) if w > 1 else t.reshape(-1)  # noqa: E731
-    kept = _ops.RenderKept(xys, depths, radii, conics, cum,
-                           _ops.KeptSort(ids, pos, bins, ctx.num_intersects, recs, order))
+    items, bins_rows, M, capacity = ctx.kept
+    kept = _ops.RenderKept(items, bins_rows, True, work, lists, M, capacity)
     kind, target, image, v_loss = loss if loss is not None else (0, None, None, None)
     gm, gs, gq, gc, go, gv, gt = _ops.render_bwd(
         flat(means, 3), flat(scales, 3), flat(quats, 4), flat(colors, 3), flat(opac, 1),
@@ -117,19 +120,19 @@ def _backward(ctx, v_img, v_depth, loss=None):
 
     def rows_of(g: torch.Tensor, like: torch.Tensor, w: int) -> torch.Tensor:
         if g.numel() == like.numel():  # batched, one image, or folded by the library
-            return g.reshape(like.shape)
+            return _shaped(g, like.shape)
         g = g.reshape(B, n, w) if w > 1 else g.reshape(B, n)
         return g.sum(0).reshape(like.shape)  # shared operand: sum over the batch
 
     need = ctx.needs_input_grad
     g_view = None
     if need[5]:
-        g_view = gv.reshape(B, 4, 4)
-        g_view = g_view.reshape(viewmat.shape) if viewmat.ndim == 3 else g_view.sum(0)
+        g_view = gv.reshape(viewmat.shape) if viewmat.ndim == 3 or B == 1 else \
+            gv.reshape(B, 4, 4).sum(0)
     g_tf = None
     if has_tf and need[7]:
-        g_tf = gt.reshape(B, K, 4, 4)
-        g_tf = g_tf.reshape(transforms.shape) if transforms.ndim == 4 else g_tf.sum(0)
+        g_tf = gt.reshape(transforms.shape) if transforms.ndim == 4 or B == 1 else \
+            gt.reshape(B, K, 4, 4).sum(0)
     return (rows_of(gm, means, 3) if need[0] else None,
             rows_of(gs, scales, 3) if need[1] else None,
             rows_of(gq, quats, 4) if need[2] else None,
@@ -159,7 +162,7 @@ class _RenderFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, v_img, v_depth):
-        gm, gs, gq, gc, go, gv, gt = _backward(ctx, v_img, v_depth)
+        gm, gs, gq, gc, go, gv, gt = _backward(ctx, ctx.saved_tensors, v_img, v_depth)
         return gm, gs, gq, gc, go, gv, None, gt, None, None
 
 
@@ -184,11 +187,12 @@ class _RenderLossFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, v_loss, _v_img):
-        img, target = ctx.saved_tensors[21:]
         if v_loss is None:
             return (None,) * 12
+        saved = ctx.saved_tensors
+        img, target = saved[13:]
         v_loss = v_loss.to(torch.float32).contiguous()
-        gm, gs, gq, gc, go, gv, gt = _backward(ctx, None, None,
+        gm, gs, gq, gc, go, gv, gt = _backward(ctx, saved, None, None,
                                                loss=(ctx.kind, target, img, v_loss))
         return gm, gs, gq, gc, go, gv, None, gt, None, None, None, None
 
@@ -254,8 +258,8 @@ def render(means3d: torch.Tensor, scales: torch.Tensor, quats: torch.Tensor,
         img, depth = _RenderFn.apply(*ops[:7], ops[7], tf_ids, statics)
     else:  # no backward can follow: the forward alone, keeping no emission positions
         img, _, _, _, depth = _fused_forward(*ops, tf_ids, statics, backward=False)
-    img = img.reshape(*S, H, W, 3)
-    return img, (depth.reshape(*S, H, W) if render_depth else None)
+    img = _shaped(img, (*S, H, W, 3))
+    return img, (_shaped(depth, (*S, H, W)) if render_depth else None)
 
 
 _LOSS_KINDS = {"l1": _ops.LOSS_L1, "mse": _ops.LOSS_MSE}
@@ -291,7 +295,7 @@ def render_loss(means3d: torch.Tensor, scales: torch.Tensor, quats: torch.Tensor
         value = torch.empty((), device=means3d.device, dtype=torch.float32)
         img = _fused_forward(*ops, tf_ids, statics, backward=False,
                              loss=(_LOSS_KINDS[loss], tgt, value))[0]
-    return value, img.reshape(*S, H, W, 3)
+    return value, _shaped(img, (*S, H, W, 3))
 
 
 def render_log(means3d: torch.Tensor, log_scales: torch.Tensor, quats: torch.Tensor,

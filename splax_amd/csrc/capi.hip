@@ -97,13 +97,14 @@ int DeviceScratch::ensure_base() {
     if (rc) return rc;
     chunk_sums_cap = 4096;
     void* h = nullptr;
-    if (hipHostMalloc(&h, sizeof(int32_t), hipHostMallocDefault) != hipSuccess)
+    if (hipHostMalloc(&h, sizeof(uint64_t), hipHostMallocDefault) != hipSuccess)
         return fail(kErrAlloc, "pinned readback allocation failed");
-    pinned_count = static_cast<int32_t*>(h);
+    pinned_count = static_cast<uint64_t*>(h);
+    *pinned_count = 0;
     void* hd = nullptr;
     if (hipHostGetDevicePointer(&hd, h, 0) != hipSuccess || !hd)
         return fail(kErrAlloc, "pinned readback mapping failed");
-    pinned_count_dev = static_cast<int32_t*>(hd);
+    pinned_count_dev = static_cast<uint64_t*>(hd);
     if (hipEventCreateWithFlags(&count_event, hipEventDisableTiming) != hipSuccess)
         return fail(kErrRuntime, "event creation failed");
     int cus = 0;
@@ -873,7 +874,7 @@ static int rasterize_fwd_core(hipStream_t s, DeviceScratch& sc, const RasterInpu
     if (rc) return fail(rc, "blend_fwd launch failed");
     if (deferred) {
         int64_t count = 0;
-        rc = settle_count(sc, tgt->capacity, &count);
+        rc = settle_count(sc, tgt->capacity, tgt->count_tag, s, &count);
         if (num_intersects) *num_intersects = count;
         return rc;
     }
@@ -1207,6 +1208,8 @@ int splat_render_fwd(splat_stream_t stream, const float* means3d, int64_t rows_m
     int32_t* count_word = reinterpret_cast<int32_t*>(sc.tickets + kCountWord);
     f.count_word = chunks > 1 ? count_word : nullptr;
     f.count_host = chunks > 1 ? sc.pinned_count_dev : nullptr;
+    if (++sc.count_tag == 0) sc.count_tag = 1;  // 0 means no tag
+    f.count_tag = sc.count_tag;
     g_last_error.clear();
     {
         StageTimer tm(s, kStageProject);
@@ -1223,7 +1226,7 @@ int splat_render_fwd(splat_stream_t stream, const float* means3d, int64_t rows_m
         tgt.chunk_prefix = sc.chunk_sums;
         tgt.num_tiles_hit = num_tiles_hit;
         tgt.count_src = count_word;
-        tgt.count_on_host = true;
+        tgt.count_tag = f.count_tag;
     }
     PixelLoss lp;
     lp.kind = loss_kind;

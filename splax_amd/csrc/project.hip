@@ -329,15 +329,16 @@ constexpr int kChunkScanThreads = 1024;
 // (1) block 0 (when chunks > 1) turns the chunk totals into exclusive prefixes, which
 //     chunk_offset_kernel (or, on the render path, the emission) then adds to the chunks' items,
 //     and with total_out non-null writes the grand total (the intersection count) there, and
-//     with total_host non-null also into that host-visible word (a system-scope store, so the
-//     host reads it once the kernel's completion is signalled, with no copy launch);
+//     with total_host non-null also into that host-visible word under host_tag (one 64-bit
+//     system-scope store, which the host polls for: no copy launch and no event, whose barrier
+//     packet every forward paid for);
 // (2) with mm non-null, block b < images folds the fused projection's per-chunk depth-range
 //     partials of image b into the image's range of visible items (what minmax_partial_kernel /
 //     minmax_final_kernel give): chunk c holds items [1024 c, 1024 c + 1024), its slot 0 the
 //     image of its first item, slot 1 the next.
 __global__ void __launch_bounds__(kChunkScanThreads)
 chunk_scan_kernel(uint32_t* sums, int64_t chunks, const uint32_t* partial, int32_t n, float* mm,
-                  int64_t images, int32_t* total_out, int32_t* total_host) {
+                  int64_t images, int32_t* total_out, uint64_t* total_host, uint32_t host_tag) {
     __shared__ uint32_t s_wave[kChunkScanThreads / 64];
     __shared__ uint32_t s_lo[kChunkScanThreads / 64], s_hi[kChunkScanThreads / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -382,7 +383,7 @@ chunk_scan_kernel(uint32_t* sums, int64_t chunks, const uint32_t* partial, int32
         // wrap-around on overflow is kept, as in cum_tiles_hit
         if (total_out && tid == kChunkScanThreads - 1) *total_out = (int32_t)run;
         if (total_host && tid == kChunkScanThreads - 1)
-            __hip_atomic_store(total_host, (int32_t)run, __ATOMIC_RELAXED,
+            __hip_atomic_store(total_host, ((uint64_t)host_tag << 32) | run, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_SYSTEM);
     }
     if (mm != nullptr && (int64_t)blockIdx.x < images) {
@@ -900,7 +901,7 @@ int launch_project_fwd_impl(const ProjectArgs& a, uint32_t* chunk_sums, const Fu
                            dim3(kChunkScanThreads), 0, stream, P.chunk_sums, blocks,
                            f ? f->mm_partial : nullptr, a.n, images > 0 ? f->depth_mm : nullptr,
                            images, offsets_later ? f->count_word : nullptr,
-                           offsets_later ? f->count_host : nullptr);
+                           offsets_later ? f->count_host : nullptr, f ? f->count_tag : 0u);
     if (blocks > 1 && !offsets_later)
         return launch_chunk_offsets(P.cum_tiles_hit, a.total, P.chunk_sums, stream);
     return hipGetLastError() == hipSuccess ? 0 : kErrLaunch;

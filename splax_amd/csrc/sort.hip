@@ -23,6 +23,8 @@
 // (image and tile fields), which the last two passes and the bin edges move, unless the caller
 // returns the sorted keys. A capacity-bounded caller need not know the count: the kernels then
 // read it from device memory (live_count) and the grids cover the capacity.
+#include <thread>
+
 #include "splat_common.hpp"
 #include "splat_internal.hpp"
 
@@ -789,19 +791,19 @@ int run_sort_and_bin(const RasterInputs& in, DeviceScratch& sc, hipStream_t stre
         return fill_zero_i32(bins, 2 * nbins, stream);
     }
     // The one device-to-host read: the intersection count (skipped when the caller supplies it).
-    // The copy is enqueued first (on the render path the chunk scan has already stored the count
-    // into the pinned word, so only the event is recorded); the depth range launches run while
-    // the host waits
+    // The copy is enqueued first (on the render path the chunk scan stores the count into the
+    // pinned word itself); the depth range launches run while the host waits
     // (splax/_rasterize/_sort/_sort.py:71-96). With a capacity-bounded target the host does not
     // wait here at all: every launch below is sized by the capacity and bounded on the device by
     // the count itself (live_count), and the caller settles the count after its last launch
     // (settle_count), so the host never stalls the stream between the projection and the blend.
     const bool deferred = !known && tgt && tgt->capacity >= 0;
     const int32_t* count_src = tgt && tgt->count_src ? tgt->count_src : in.cum + (total - 1);
-    const bool on_host = tgt && tgt->count_on_host;  // already stored by its kernel
-    if (!known && ((!on_host && hipMemcpyAsync(sc.pinned_count, count_src, sizeof(int32_t),
-                                               hipMemcpyDeviceToHost, stream) != hipSuccess) ||
-                   hipEventRecord(sc.count_event, stream) != hipSuccess))
+    const bool on_host = tgt && tgt->count_tag != 0;  // stored by its kernel
+    if (!known && !on_host &&
+        (hipMemcpyAsync(sc.pinned_count, count_src, sizeof(int32_t), hipMemcpyDeviceToHost,
+                        stream) != hipSuccess ||
+         hipEventRecord(sc.count_event, stream) != hipSuccess))
         return fail(kErrRuntime, "count readback enqueue failed");
     const float* depth_mm = sc.depth_mm;
     if (!wide && tgt && tgt->depth_mm) {
@@ -831,7 +833,7 @@ int run_sort_and_bin(const RasterInputs& in, DeviceScratch& sc, hipStream_t stre
     } else {
         if (hipEventSynchronize(sc.count_event) != hipSuccess)
             return fail(kErrRuntime, "count readback failed");
-        M = *sc.pinned_count;
+        M = (int32_t)(uint32_t)*sc.pinned_count;
     }
     if (!deferred) {
         if (M < 0) return fail(kErrTooMany, "intersection count overflowed int32");
@@ -974,10 +976,39 @@ int run_sort_and_bin(const RasterInputs& in, DeviceScratch& sc, hipStream_t stre
     return 0;
 }
 
-int settle_count(DeviceScratch& sc, int64_t capacity, int64_t* M_out) {
-    if (hipEventSynchronize(sc.count_event) != hipSuccess)
-        return fail(kErrRuntime, "count readback failed");
-    const int64_t M = *sc.pinned_count;
+// Waits for the pinned word to carry `tag`. The word is polled (the count is there some
+// microseconds before an event's signal would be); a stream that drained or failed without
+// storing it is an error, so the wait always ends.
+static int wait_tagged_count(DeviceScratch& sc, uint32_t tag, hipStream_t stream, uint64_t* word) {
+    for (bool drained = false;; std::this_thread::yield()) {
+        for (int k = 0; k < 512; ++k) {
+            *word = __atomic_load_n(sc.pinned_count, __ATOMIC_ACQUIRE);
+            if ((uint32_t)(*word >> 32) == tag) return 0;
+            __builtin_ia32_pause();
+        }
+        if (drained) return fail(kErrRuntime, "the intersection count was not stored");
+        const hipError_t e = hipStreamQuery(stream);
+        if (e == hipErrorNotReady)
+            (void)hipGetLastError();
+        else if (e == hipSuccess)
+            drained = true;  // everything the stream held has run: one last look
+        else
+            return fail(kErrRuntime, std::string("count readback failed: ") + hipGetErrorString(e));
+    }
+}
+
+int settle_count(DeviceScratch& sc, int64_t capacity, uint32_t tag, hipStream_t stream,
+                 int64_t* M_out) {
+    uint64_t word = 0;
+    if (tag) {
+        const int rc = wait_tagged_count(sc, tag, stream, &word);
+        if (rc) return rc;
+    } else {
+        if (hipEventSynchronize(sc.count_event) != hipSuccess)
+            return fail(kErrRuntime, "count readback failed");
+        word = *sc.pinned_count;
+    }
+    const int64_t M = (int32_t)(uint32_t)word;
     *M_out = M;
     if (M < 0) return fail(kErrTooMany, "intersection count overflowed int32");
     sc.last_count = M;

@@ -140,8 +140,11 @@ struct DeviceScratch {
     int32_t* tile_bins = nullptr; int64_t bins_cap = 0;             // (start, end) pairs
     float* depth_mm = nullptr; int64_t mm_cap = 0;                  // 2 * B
     uint32_t* mm_partial = nullptr; int64_t mm_partial_cap = 0;     // 2 * blocks
-    int32_t* pinned_count = nullptr;
-    int32_t* pinned_count_dev = nullptr;  // the device's address of pinned_count
+    // the intersection count's readback word: the count in the low half and, when a kernel stores
+    // it, the call's tag in the high half
+    uint64_t* pinned_count = nullptr;
+    uint64_t* pinned_count_dev = nullptr;  // the device's address of pinned_count
+    uint32_t count_tag = 0;                // the last tag given out
     hipEvent_t count_event = nullptr;
     int64_t last_count = -1;  // the last settled deferred count: the sort's partition shape
     // Calls on one device share these buffers: a call on another stream than the last user's
@@ -238,9 +241,10 @@ struct FusedRecords {
     // projection leaves cum_tiles_hit chunk-local (chunk_sums then hold the chunks' exclusive
     // prefixes): the emission adds them (SortTargets::chunk_prefix)
     int32_t* count_word = nullptr;
-    // non-null (with count_word): the chunk scan also stores the count into this host-visible
-    // word (DeviceScratch::pinned_count_dev), so the readback needs no copy
-    int32_t* count_host = nullptr;
+    // non-null (with count_word): the chunk scan also stores the count, tagged, into this
+    // host-visible word (DeviceScratch::pinned_count_dev), so the readback needs no copy
+    uint64_t* count_host = nullptr;
+    uint32_t count_tag = 0;
 };
 int launch_project_fwd_fused(const ProjectArgs& a, const FusedRecords& f, DeviceScratch& sc,
                              hipStream_t stream);
@@ -278,9 +282,9 @@ struct SortTargets {
     const uint32_t* chunk_prefix = nullptr;
     const int32_t* num_tiles_hit = nullptr;
     const int32_t* count_src = nullptr;
-    // the kernel that forms count_src also stores it into the pinned readback word
-    // (FusedRecords::count_host): only the readback event is recorded
-    bool count_on_host = false;
+    // nonzero: the kernel that forms count_src also stores it into the pinned readback word with
+    // this tag (FusedRecords::count_host), and the host waits for the tag
+    uint32_t count_tag = 0;
 };
 
 // Where sort_and_bin left its results: sorted keys (int32 when packed, uint64 when wide), ids,
@@ -303,7 +307,8 @@ int run_sort_and_bin(const RasterInputs& in, DeviceScratch& sc, hipStream_t stre
                      SortOutputs* out, bool full_keys = false);
 // Waits for the deferred count's readback (enqueued after the projection, so normally long
 // complete), reports it in *M_out and fails with kErrTooMany above the capacity.
-int settle_count(DeviceScratch& sc, int64_t capacity, int64_t* M_out);
+int settle_count(DeviceScratch& sc, int64_t capacity, uint32_t tag, hipStream_t stream,
+                 int64_t* M_out);
 
 // Writes the packed blend record (4 float4) of each of the in.B_geom * in.n geometry items.
 int launch_pack_records(const RasterInputs& in, float4* recs, hipStream_t stream);

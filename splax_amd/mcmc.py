@@ -54,7 +54,7 @@ def compute_relocation(opacities: torch.Tensor, scales: torch.Tensor, ratios: to
     dev = _lib.require_gpu(opac, sc, rat)
     new_o = torch.empty_like(opac)
     new_s = torch.empty_like(sc)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().splat_mcmc_compute_relocation(
             _lib.stream_handle(dev), _lib.ptr(opac), _lib.ptr(sc), _lib.ptr(rat), n,
             _n_max(binoms), _lib.ptr(new_o), _lib.ptr(new_s))
@@ -87,7 +87,7 @@ def relocate_(key: int, means3d: torch.Tensor, log_scales: torch.Tensor, quats: 
     dev = _lib.require_gpu(*arrays)
     reset = torch.empty((n,), device=dev, dtype=torch.bool)
     source = torch.empty((n,), device=dev, dtype=torch.int32) if return_source else None
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().splat_mcmc_relocate(
             _lib.stream_handle(dev), *(_lib.ptr(t) for t in arrays), n, _n_max(binoms),
             float(min_opacity), int(key) & 0xFFFFFFFFFFFFFFFF, _lib.ptr(source), _lib.ptr(reset))
@@ -112,7 +112,7 @@ def relocate(key: int, means3d: torch.Tensor, log_scales: torch.Tensor, quats: t
     dev = _lib.require_gpu(*arrays)
     new = tuple(torch.empty_like(t) for t in arrays)
     reset = torch.empty((n,), device=dev, dtype=torch.bool)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().splat_mcmc_relocate_copy(
             _lib.stream_handle(dev), *(_lib.ptr(t) for t in arrays), n, _n_max(binoms),
             float(min_opacity), int(key) & 0xFFFFFFFFFFFFFFFF, *(_lib.ptr(t) for t in new),
@@ -154,7 +154,7 @@ def inject_noise(key: int, means3d: torch.Tensor, log_scales: torch.Tensor, quat
     dev = _lib.require_gpu(m, ls, q, lo, *(() if z is None else (z,)))
     if out is None:
         out = torch.empty_like(m)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.lib().splat_mcmc_inject_noise(
             _lib.stream_handle(dev), _lib.ptr(m), _lib.ptr(ls), _lib.ptr(q), _lib.ptr(lo), n,
             float(scaler), float(min_opacity), int(key) & 0xFFFFFFFFFFFFFFFF,

@@ -91,7 +91,7 @@ class Adam:
                 raise ValueError(f"maps name groups {sorted(unknown)} that do not exist")
             map_arr = (ctypes.c_int32 * len(arr))(*[int(maps.get(k, MAP_NONE))
                                                     for k in self.params])
-        with torch.cuda.device(self._dev):
+        with _lib.on_device(self._dev):
             st = _lib.lib().splat_adam_step_mapped(
                 _lib.stream_handle(self._dev), ctypes.addressof(arr), len(arr),
                 None if map_arr is None else ctypes.addressof(map_arr), self.b1, self.b2,
@@ -106,7 +106,7 @@ class Adam:
         mask = reset.contiguous()
         mask = mask.view(torch.uint8) if mask.dtype == torch.bool else mask.to(torch.uint8)
         arr, _ = self._groups(None, self.count)
-        with torch.cuda.device(self._dev):
+        with _lib.on_device(self._dev):
             st = _lib.lib().splat_adam_reset_rows(
                 _lib.stream_handle(self._dev), ctypes.addressof(arr), len(arr), mask.data_ptr(), rows)
         _lib.check(st, "adam_reset_rows")

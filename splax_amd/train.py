@@ -70,7 +70,7 @@ class _PixelLossFn(torch.autograd.Function):
         partials = torch.empty(((count + 4095) // 4096,), device=dev, dtype=torch.float64)
         loss = torch.empty((), device=dev, dtype=torch.float32)
         fwd = getattr(_lib.lib(), f"splat_{kind}_loss_fwd")
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             st = fwd(_lib.stream_handle(dev), img.data_ptr(), target.data_ptr(), count,
                      partials.data_ptr(), loss.data_ptr())
         _lib.check(st, f"{kind}_loss_fwd")
@@ -84,7 +84,7 @@ class _PixelLossFn(torch.autograd.Function):
         v_loss = v_loss.to(torch.float32).contiguous()
         v_img = torch.empty_like(img)
         bwd = getattr(_lib.lib(), f"splat_{ctx.kind}_loss_bwd")
-        with torch.cuda.device(img.device):
+        with _lib.on_device(img.device):
             st = bwd(_lib.stream_handle(img.device), img.data_ptr(), target.data_ptr(),
                      img.numel(), v_loss.data_ptr(), v_img.data_ptr())
         _lib.check(st, f"{ctx.kind}_loss_bwd")
