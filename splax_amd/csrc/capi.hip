@@ -178,11 +178,14 @@ int DeviceScratch::ensure_sort(int64_t M, int64_t bins, int32_t B, bool wide) {
         if (rc) return rc;
         wide_cap = cap;
     }
-    const int64_t parts = (M + kSortTileMin - 1) / kSortTileMin;
-    if (parts * 256 > part_counts_cap) {
+    // digit counts: one pass's partitions, or for a small sort those of every pass
+    int64_t count_rows = (M + kSortTileMin - 1) / kSortTileMin;
+    if (M <= kSortSmallM)
+        count_rows = kMaxPasses * ((M + kSortSmallTile - 1) / kSortSmallTile);
+    if (count_rows * 256 > part_counts_cap) {
         sync_once();
         dev_free(&part_counts);
-        int64_t cap = (int64_t)(parts * 1.25 + 1) * 256;
+        int64_t cap = (int64_t)(count_rows * 1.25 + 1) * 256;
         rc = dev_alloc(&part_counts, cap, false);
         if (rc) {
             part_counts_cap = 0;
@@ -1190,7 +1193,7 @@ int splat_render_fwd(splat_stream_t stream, const float* means3d, int64_t rows_m
     if (L.overflow) return fail(kErrKeyOverflow, "render_fwd: intersection key overflow");
     sc.workload(B, num_gaussians, L.num_tiles);
     // the depth range from the projection: packed key, chunks meeting at most two images
-    const bool fuse_range = L.packed && num_gaussians >= 1024;
+    const bool fuse_range = L.packed && num_gaussians >= project_fwd_chunk_items(total);
     const int64_t chunks = project_fwd_chunks(total);
     {
         const int32_t bpi = (num_gaussians + 4095) / 4096;

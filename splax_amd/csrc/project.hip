@@ -2,7 +2,7 @@
 // backward, gfx950.
 //
 // project_fwd: one thread per flat item (image b, gaussian g), restating _project_kernel
-// (splax/_project/_kernels.py:122-248). Each workgroup owns a contiguous chunk of 1024 items;
+// (splax/_project/_kernels.py:122-248). Each workgroup owns a contiguous chunk of 1024 (or 256) items;
 // after counting tiles it scans its chunk in LDS, writes the chunk-local inclusive prefix to
 // cum_tiles_hit and the chunk's total to a partials array. One workgroup then scans the
 // partials, and a last pass adds each chunk's offset, which gives the global inclusive scan the
@@ -46,9 +46,16 @@ struct ProjectParams {
 };
 
 constexpr int kProjThreads = 256;
-// Items per chunk of the projection's tile-count scan (one forward workgroup each): 1024 keeps the
-// chunk-total scan short (about 12 totals per scan thread at 12M items).
-constexpr int kProjFwdThreads = 1024;
+// Items per chunk of the projection's tile-count scan (one forward workgroup each, one item per
+// thread): 1024 keeps the chunk-total scan short (about 12 totals per scan thread at 12M items).
+// Up to kProjSmallItems items the chunks hold 256: with 1024 they would be fewer than the CUs, and
+// the projection is bound by VALU issue on the CUs it runs on (10K items are 10 workgroups of
+// 1024, 10.0 us, or 40 of 256, 6.5 us; 100K items 13.9 and 11.7 us).
+constexpr int kProjChunkBig = 1024, kProjChunkSmall = 256;
+constexpr int64_t kProjSmallItems = 256 * kProjChunkBig;
+int32_t project_fwd_chunk_items(int64_t total) {
+    return total <= kProjSmallItems ? kProjChunkSmall : kProjChunkBig;
+}
 
 __device__ __forceinline__ bool apply_transform(const float* transforms, int32_t image_id,
                                                 int32_t num_transforms, bool sel_tf,
@@ -221,21 +228,17 @@ __device__ __forceinline__ ItemOut project_item(const ProjectParams& P, int64_t 
     return ItemOut{count, xy.x, xy.y, depth, con0, con1, con2, opac};
 }
 
-// Items per thread of the fused projection + scan; one workgroup covers 256 * kProjItems items.
-// One item per thread keeps the loads coalesced and gives the latency-bound projection the most
-// waves in flight.
-constexpr int kProjItems = 1;
-static_assert(kProjFwdThreads * kProjItems == kProjChunkItems, "one chunk per projection workgroup");
-
 // kFused (the fused render forward): also the item's packed blend record and the chunk's depth
-// range partials (the chunk spans at most two images: num_gaussians >= 1024).
-template <bool kFused>
-__global__ void __launch_bounds__(kProjFwdThreads) project_fwd_kernel(ProjectParams P) {
-    __shared__ int32_t s_wave[kProjFwdThreads / 64];
-    __shared__ uint32_t s_mm[kProjFwdThreads / 64][4];
+// range partials (the chunk spans at most two images: num_gaussians >= kThreads). One item per
+// thread keeps the loads coalesced and gives the projection the most waves in flight.
+template <bool kFused, int kThreads>
+__global__ void __launch_bounds__(kThreads) project_fwd_kernel(ProjectParams P) {
+    constexpr int kProjItems = 1;
+    __shared__ int32_t s_wave[kThreads / 64];
+    __shared__ uint32_t s_mm[kThreads / 64][4];
     const int tid = threadIdx.x;
     const uint32_t part = blockIdx.x;
-    const int64_t base = (int64_t)part * (kProjFwdThreads * kProjItems);
+    const int64_t base = (int64_t)part * (kThreads * kProjItems);
     // Items are blocked per thread (thread t owns base + t*K .. +K-1) so the per-thread running
     // sum plus one block scan gives the inclusive prefix.
     int32_t cnt[kProjItems];
@@ -261,7 +264,7 @@ __global__ void __launch_bounds__(kProjFwdThreads) project_fwd_kernel(ProjectPar
 #pragma unroll
                 for (int q = 0; q < 4; ++q) dst[q] = r[q];
                 // visible items (radii > 0) set the range, splax/_rasterize/_sort/_kernels.py:38-73;
-                // slot 0 or 1: with n >= 1024 a chunk meets at most two images
+                // slot 0 or 1: with n >= kThreads a chunk meets at most two images
                 if (P.mm_partial && o.count > 0) {
                     const bool second = idx / P.n != base / P.n;
                     const uint32_t u = f2ord(o.depth);
@@ -297,7 +300,7 @@ __global__ void __launch_bounds__(kProjFwdThreads) project_fwd_kernel(ProjectPar
         if (P.mm_partial && tid < 4) {
             uint32_t v = s_mm[0][tid];
 #pragma unroll
-            for (int w = 1; w < kProjFwdThreads / 64; ++w) {
+            for (int w = 1; w < kThreads / 64; ++w) {
                 const uint32_t o = s_mm[w][tid];
                 v = (tid & 1) ? (o > v ? o : v) : (o < v ? o : v);
             }
@@ -306,7 +309,7 @@ __global__ void __launch_bounds__(kProjFwdThreads) project_fwd_kernel(ProjectPar
     }
     int32_t wave_off = 0, block_total = 0;
 #pragma unroll
-    for (int w = 0; w < kProjFwdThreads / 64; ++w) {
+    for (int w = 0; w < kThreads / 64; ++w) {
         int32_t v = s_wave[w];
         if (w < wave) wave_off += v;
         block_total += v;
@@ -334,10 +337,14 @@ constexpr int kChunkScanThreads = 1024;
 //     packet every forward paid for);
 // (2) with mm non-null, block b < images folds the fused projection's per-chunk depth-range
 //     partials of image b into the image's range of visible items (what minmax_partial_kernel /
-//     minmax_final_kernel give): chunk c holds items [1024 c, 1024 c + 1024), its slot 0 the
-//     image of its first item, slot 1 the next.
+//     minmax_final_kernel give): chunk c holds items [chunk_items c, chunk_items (c + 1)), its
+//     slot 0 the image of its first item, slot 1 the next.
+// kChunkScanPer: chunks per thread kept in registers. The launch takes the smallest of 4, 16 and
+// 64 that holds the run (64 predicated loads for one chunk each cost half of the kernel: 6.3 us
+// at 10 to 400 chunks, 3.0 to 3.6 us with 4; 13.0 and 12.3 us at 12K chunks with 16).
+template <int kChunkScanPer>
 __global__ void __launch_bounds__(kChunkScanThreads)
-chunk_scan_kernel(uint32_t* sums, int64_t chunks, const uint32_t* partial, int32_t n, float* mm,
+chunk_scan_kernel(uint32_t* sums, int64_t chunks, int32_t chunk_items, const uint32_t* partial, int32_t n, float* mm,
                   int64_t images, int32_t* total_out, uint64_t* total_host, uint32_t host_tag) {
     __shared__ uint32_t s_wave[kChunkScanThreads / 64];
     __shared__ uint32_t s_lo[kChunkScanThreads / 64], s_hi[kChunkScanThreads / 64];
@@ -348,7 +355,6 @@ chunk_scan_kernel(uint32_t* sums, int64_t chunks, const uint32_t* partial, int32
         const int64_t hi = lo + per < chunks ? lo + per : chunks;
         // runs of up to kChunkScanPer chunks (up to 64Ki chunks, 67M items) are loaded into
         // registers at once, so their load latencies overlap; longer runs take a sequential loop
-        constexpr int kChunkScanPer = 64;
         const bool in_regs = per <= kChunkScanPer;
         uint32_t v[kChunkScanPer];
         uint32_t total = 0;
@@ -388,12 +394,12 @@ chunk_scan_kernel(uint32_t* sums, int64_t chunks, const uint32_t* partial, int32
     }
     if (mm != nullptr && (int64_t)blockIdx.x < images) {
         const int64_t image = blockIdx.x;
-        const int64_t c0 = image * n / kProjFwdThreads;
-        int64_t c1 = ((image + 1) * n - 1) / kProjFwdThreads;
+        const int64_t c0 = image * n / chunk_items;
+        int64_t c1 = ((image + 1) * n - 1) / chunk_items;
         c1 = c1 < chunks - 1 ? c1 : chunks - 1;
         uint32_t lo = 0xffffffffu, hi = 0u;
         for (int64_t c = c0 + tid; c <= c1; c += kChunkScanThreads) {
-            const int64_t slot = image - c * kProjFwdThreads / n;  // 0 or 1
+            const int64_t slot = image - c * chunk_items / n;  // 0 or 1
             const uint32_t x = partial[4 * c + 2 * slot], y = partial[4 * c + 2 * slot + 1];
             lo = x < lo ? x : lo;
             hi = y > hi ? y : hi;
@@ -422,11 +428,10 @@ chunk_scan_kernel(uint32_t* sums, int64_t chunks, const uint32_t* partial, int32
 
 // cum_tiles_hit += the chunk's offset (chunk 0 has none); int32 wrap-around on overflow is kept,
 // the host reports a negative total as too many intersections. A chunk is one workgroup of the
-// projection, one item per thread.
-static_assert(kProjItems == 1, "chunk_offset_kernel maps one thread to one item");
-__global__ void __launch_bounds__(kProjFwdThreads) chunk_offset_kernel(int32_t* cum, int64_t total,
-                                                           const uint32_t* offsets) {
-    const int64_t idx = (int64_t)(blockIdx.x + 1) * kProjFwdThreads + threadIdx.x;
+// projection and one of this kernel, one item per thread.
+__global__ void __launch_bounds__(kProjChunkBig) chunk_offset_kernel(int32_t* cum, int64_t total,
+                                                                     const uint32_t* offsets) {
+    const int64_t idx = (int64_t)(blockIdx.x + 1) * blockDim.x + threadIdx.x;
     if (idx < total) cum[idx] = (int32_t)((uint32_t)cum[idx] + offsets[blockIdx.x + 1]);
 }
 
@@ -834,7 +839,7 @@ viewmat_reduce_kernel(const float* partials, int32_t blocks_per_image, float* v_
 
 // Chunks (workgroups) of a projection over `total` items: one chunk total of scratch each.
 int64_t project_fwd_chunks(int64_t total) {
-    const int64_t per_block = (int64_t)kProjFwdThreads * kProjItems;
+    const int64_t per_block = project_fwd_chunk_items(total);
     return (total + per_block - 1) / per_block;
 }
 
@@ -889,19 +894,37 @@ int launch_project_fwd_impl(const ProjectArgs& a, uint32_t* chunk_sums, const Fu
     P.mm_partial = f ? f->mm_partial : nullptr;
     // the render path leaves the chunk offsets to the emission when there are several chunks
     const bool offsets_later = f && f->count_word && blocks > 1;
-    if (f)
-        hipLaunchKernelGGL(project_fwd_kernel<true>, dim3((unsigned)blocks),
-                           dim3(kProjFwdThreads), 0, stream, P);
+    const int32_t chunk = project_fwd_chunk_items(a.total);
+    const dim3 grid((unsigned)blocks), block(chunk);
+    if (f && chunk == kProjChunkSmall)
+        hipLaunchKernelGGL((project_fwd_kernel<true, kProjChunkSmall>), grid, block, 0, stream, P);
+    else if (f)
+        hipLaunchKernelGGL((project_fwd_kernel<true, kProjChunkBig>), grid, block, 0, stream, P);
+    else if (chunk == kProjChunkSmall)
+        hipLaunchKernelGGL((project_fwd_kernel<false, kProjChunkSmall>), grid, block, 0, stream, P);
     else
-        hipLaunchKernelGGL(project_fwd_kernel<false>, dim3((unsigned)blocks),
-                           dim3(kProjFwdThreads), 0, stream, P);
+        hipLaunchKernelGGL((project_fwd_kernel<false, kProjChunkBig>), grid, block, 0, stream, P);
     const int64_t images = (f && f->depth_mm) ? a.total / a.n : 0;
-    if (blocks > 1 || images > 0)
-        hipLaunchKernelGGL(chunk_scan_kernel, dim3((unsigned)(images > 1 ? images : 1)),
-                           dim3(kChunkScanThreads), 0, stream, P.chunk_sums, blocks,
-                           f ? f->mm_partial : nullptr, a.n, images > 0 ? f->depth_mm : nullptr,
-                           images, offsets_later ? f->count_word : nullptr,
-                           offsets_later ? f->count_host : nullptr, f ? f->count_tag : 0u);
+    if (blocks > 1 || images > 0) {
+        const dim3 scan_grid((unsigned)(images > 1 ? images : 1)), scan_block(kChunkScanThreads);
+        const uint32_t* mm_partial = f ? f->mm_partial : nullptr;
+        float* mm = images > 0 ? f->depth_mm : nullptr;
+        int32_t* count = offsets_later ? f->count_word : nullptr;
+        uint64_t* host = offsets_later ? f->count_host : nullptr;
+        const uint32_t tag = f ? f->count_tag : 0u;
+        if (blocks <= 4 * kChunkScanThreads)
+            hipLaunchKernelGGL(chunk_scan_kernel<4>, scan_grid, scan_block, 0, stream,
+                               P.chunk_sums, blocks, chunk, mm_partial, a.n, mm, images, count,
+                               host, tag);
+        else if (blocks <= 16 * kChunkScanThreads)
+            hipLaunchKernelGGL(chunk_scan_kernel<16>, scan_grid, scan_block, 0, stream,
+                               P.chunk_sums, blocks, chunk, mm_partial, a.n, mm, images, count,
+                               host, tag);
+        else
+            hipLaunchKernelGGL(chunk_scan_kernel<64>, scan_grid, scan_block, 0, stream,
+                               P.chunk_sums, blocks, chunk, mm_partial, a.n, mm, images, count,
+                               host, tag);
+    }
     if (blocks > 1 && !offsets_later)
         return launch_chunk_offsets(P.cum_tiles_hit, a.total, P.chunk_sums, stream);
     return hipGetLastError() == hipSuccess ? 0 : kErrLaunch;
@@ -911,8 +934,9 @@ int launch_chunk_offsets(int32_t* cum, int64_t total, const uint32_t* chunk_pref
                          hipStream_t stream) {
     const int64_t blocks = project_fwd_chunks(total);
     if (blocks > 1)
-        hipLaunchKernelGGL(chunk_offset_kernel, dim3((unsigned)(blocks - 1)), dim3(kProjFwdThreads),
-                           0, stream, cum, total, chunk_prefix);
+        hipLaunchKernelGGL(chunk_offset_kernel, dim3((unsigned)(blocks - 1)),
+                           dim3(project_fwd_chunk_items(total)), 0, stream, cum, total,
+                           chunk_prefix);
     return hipGetLastError() == hipSuccess ? 0 : kErrLaunch;
 }
 
@@ -988,7 +1012,7 @@ static uint32_t* g_noalloc_scratch[kNoAllocDevices] = {};
 int launch_project_fwd_noalloc(const ProjectArgs& a, hipStream_t stream) {
     if (project_fwd_chunks(a.total) > kNoAllocMaxChunks)
         return fail(kErrArgs, "project_fwd_noalloc: more than " +
-                                  std::to_string(kNoAllocMaxChunks * kProjFwdThreads) +
+                                  std::to_string(kNoAllocMaxChunks * kProjChunkBig) +
                                   " items (the fixed scratch holds " +
                                   std::to_string(kNoAllocMaxChunks) + " chunk totals)");
     int dev = -1;

@@ -139,6 +139,7 @@ struct EmitParams {
     // the render path: cum is chunk-local, finalized here (cum_fix, the same array) from each
     // chunk's exclusive prefix; nth holds the items' own counts
     const uint32_t* chunk_prefix; const int32_t* nth; int32_t* cum_fix;
+    int32_t chunk_shift;  // log2 of project_fwd_chunk_items
     int32_t tiles_x, tiles_y, tile_bits, depth_bits;
     void* keys; int32_t* owner;
 };
@@ -161,7 +162,7 @@ __global__ void __launch_bounds__(256) emit_keys_kernel(EmitParams P) {
         fin_raw = P.cum_fix[idx];
         nth = P.nth[idx];
     }
-    const uint32_t cpre = P.chunk_prefix ? P.chunk_prefix[idx / kProjChunkItems] : 0u;
+    const uint32_t cpre = P.chunk_prefix ? P.chunk_prefix[idx >> P.chunk_shift] : 0u;
     const int32_t prev = (!P.chunk_prefix && idx > 0) ? P.cum[idx - 1] : 0;
     const int32_t rad = P.radii[idx];
     const float depth = P.depths[idx];
@@ -591,6 +592,131 @@ static void launch_pass(const K* keys_in, const int32_t* vals_in, const int32_t*
                        vals_out, ids_out, M, m_dev, shift, counts, totals, parts);
 }
 
+// ------------------------------------------------------------------ small sorts
+// Up to kSortSmallM keys a pass is bound by its launches and their latency, not by bytes: 27K keys
+// took 13.9 us a pass (count 2.9, scan 2.8, scatter 8.1 and the gaps between them) over 7
+// partitions of 4096. The small sort takes 1024-key partitions (256 threads, so four times the
+// CUs and barriers of four waves), sums the partitions' digit counts inside the scatter instead
+// of in a scan launch (at most 80 per digit), and counts the next pass's digits while it writes
+// the keys (an atomic per key: 25 G/s here, 2.6 us at 64K keys, which is why the line lies there;
+// the first pass's digits take a launch of their own). One launch per pass, 6.5 to 8.2 us each, and
+// 3.6 us for the first digits.
+
+// Digit counts of the first pass, counts[part][digit]; clears the later passes' counts (`clear`)
+// and the tile bins.
+template <typename K>
+__global__ void __launch_bounds__(256)
+small_count_kernel(const K* __restrict__ keys, int64_t M_bound, const int32_t* __restrict__ m_dev,
+                   int shift, uint32_t* __restrict__ counts, uint32_t* __restrict__ clear,
+                   int64_t clear_words, int32_t* __restrict__ bins, int64_t nbins2) {
+    __shared__ uint32_t s_h[4][256];
+    const int tid = threadIdx.x, wave = tid >> 6;
+    for (int w = 0; w < 4; ++w) s_h[w][tid] = 0u;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + tid; i < clear_words; i += (int64_t)gridDim.x * 256)
+        clear[i] = 0u;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + tid; i < nbins2; i += (int64_t)gridDim.x * 256)
+        bins[i] = 0;
+    __syncthreads();
+    const int64_t M = live_count(m_dev, M_bound);
+    const int64_t base = (int64_t)blockIdx.x * kSortSmallTile;
+#pragma unroll
+    for (int i = 0; i < kSortSmallTile / 256; ++i) {
+        const int64_t pos = base + i * 256 + tid;
+        if (pos < M) atomicAdd(&s_h[wave][(uint32_t)(keys[pos] >> shift) & 255u], 1u);
+    }
+    __syncthreads();
+    counts[(int64_t)blockIdx.x * 256 + tid] = (s_h[0][tid] + s_h[1][tid]) + (s_h[2][tid] + s_h[3][tid]);
+}
+
+// Stable scatter of one 1024-key partition (as rts_scatter_kernel), its digit offsets summed from
+// counts[part][digit] of the live partitions; next_counts (null for the last pass) receives the
+// digits at next_shift of the keys it places. A key's destination is below the live count by
+// construction (every position below it is counted once).
+template <typename K, typename KO>
+__global__ void __launch_bounds__(256)
+small_scatter_kernel(const K* __restrict__ keys_in, const int32_t* __restrict__ vals_in,
+                     const int32_t* __restrict__ ids_in, KO* __restrict__ keys_out,
+                     int32_t* __restrict__ vals_out, int32_t* __restrict__ ids_out,
+                     int64_t M_bound, const int32_t* __restrict__ m_dev, int shift,
+                     const uint32_t* __restrict__ counts, uint32_t* __restrict__ next_counts,
+                     int next_shift) {
+    constexpr int kItems = kSortSmallTile / 256;
+    __shared__ uint32_t s_cnt[4][256];
+    __shared__ uint32_t s_tmp[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t M = live_count(m_dev, M_bound);
+    const int64_t base = (int64_t)blockIdx.x * kSortSmallTile;
+    if (base >= M) return;  // uniform, before any barrier
+    const int live = (int)((M + kSortSmallTile - 1) / kSortSmallTile);
+    for (int w = 0; w < 4; ++w) s_cnt[w][tid] = 0u;
+    const int64_t my0 = base + wave * (kItems * 64) + lane;
+    const int64_t rem = M - my0;
+    K key[kItems];
+    int32_t val[kItems], id[kItems];
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+        const bool in = i * 64 < rem;
+        key[i] = in ? keys_in[my0 + i * 64] : (K)~(K)0;
+        id[i] = in ? ids_in[my0 + i * 64] : 0;
+        val[i] = in && vals_out ? (vals_in ? vals_in[my0 + i * 64] : (int32_t)(my0 + i * 64)) : 0;
+    }
+    // digit tid: its keys in the partitions before this one, and in all
+    uint32_t before = 0, total = 0;
+    for (int q0 = 0; q0 < live; q0 += 16) {
+        uint32_t c[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) c[q] = q0 + q < live ? counts[(q0 + q) * 256 + tid] : 0u;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            before += q0 + q < (int)blockIdx.x ? c[q] : 0u;
+            total += c[q];
+        }
+    }
+    __syncthreads();
+    // stable per-wave ranking: lanes with equal digits found by 8 ballots
+    const uint64_t lt_mask = (1ull << lane) - 1ull;
+    uint32_t rank[kItems];
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+        const uint32_t d = (uint32_t)(key[i] >> shift) & 255u;
+        uint64_t peers = __ballot(i * 64 < rem);  // the keys past the count rank among themselves
+        peers = i * 64 < rem ? peers : ~peers;
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+            const bool bit = (d >> b) & 1u;
+            const uint64_t bal = __ballot(bit);
+            peers &= bit ? bal : ~bal;
+        }
+        const uint32_t below = (uint32_t)__popcll(peers & lt_mask);
+        const uint32_t old = s_cnt[wave][d];
+        rank[i] = old + below;
+        if (below == 0 && i * 64 < rem) s_cnt[wave][d] = old + (uint32_t)__popcll(peers);
+    }
+    const uint32_t digit_base = scan_256(total, s_tmp, nullptr) + before;  // holds the barriers
+    uint32_t run = digit_base;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {  // the wave's first destination of digit tid
+        const uint32_t c = s_cnt[w][tid];
+        s_cnt[w][tid] = run;
+        run += c;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+        if (i * 64 >= rem) continue;
+        const uint32_t dest = s_cnt[wave][(uint32_t)(key[i] >> shift) & 255u] + rank[i];
+        if constexpr (sizeof(KO) < sizeof(K))
+            keys_out[dest] = (KO)(key[i] >> 16);
+        else
+            keys_out[dest] = key[i];
+        if (vals_out) vals_out[dest] = val[i];
+        ids_out[dest] = id[i];
+        if (next_counts)
+            atomicAdd(&next_counts[(dest / kSortSmallTile) * 256 +
+                                   ((uint32_t)(key[i] >> next_shift) & 255u)], 1u);
+    }
+}
+
 // A pass over packed keys of one of three forms: 32-bit keys in and out (kind 0), 32-bit in and
 // their high halves out (kind 1), 16-bit high halves in and out (kind 2; shift counts from bit
 // 16).
@@ -874,6 +1000,7 @@ int run_sort_and_bin(const RasterInputs& in, DeviceScratch& sc, hipStream_t stre
         E.map_opac = in.map_opac; E.rows_map_opac = in.rows_map_opac;
         E.cum = in.cum; E.mm = depth_mm; E.n = in.n; E.total = total; E.M = M; E.m_dev = m_dev;
         E.chunk_prefix = chunk_prefix;
+        E.chunk_shift = 31 - __builtin_clz((unsigned)project_fwd_chunk_items(total));
         E.nth = tgt ? tgt->num_tiles_hit : nullptr;
         E.cum_fix = const_cast<int32_t*>(in.cum);
         E.tiles_x = L.tiles_x; E.tiles_y = L.tiles_y; E.tile_bits = L.tile_bits;
@@ -887,6 +1014,22 @@ int run_sort_and_bin(const RasterInputs& in, DeviceScratch& sc, hipStream_t stre
     }
     {
         StageTimer tm(stream, kStageSort);
+        const bool small = M <= kSortSmallM;
+        const int64_t small_parts = (M + kSortSmallTile - 1) / kSortSmallTile;
+        const int64_t pass_words = small_parts * 256;
+        if (small) {
+            const dim3 grid((unsigned)small_parts);
+            uint32_t* later = sc.part_counts + pass_words;
+            if (wide)
+                hipLaunchKernelGGL(small_count_kernel<uint64_t>, grid, dim3(256), 0, stream,
+                                   sc.wkeys[0], M, m_dev, ps.shift[0], sc.part_counts, later,
+                                   (ps.n - 1) * pass_words, bins, 2 * nbins);
+            else
+                hipLaunchKernelGGL(small_count_kernel<uint32_t>, grid, dim3(256), 0, stream,
+                                   reinterpret_cast<const uint32_t*>(sc.keys[0]), M, m_dev,
+                                   ps.shift[0], sc.part_counts, later, (ps.n - 1) * pass_words,
+                                   bins, 2 * nbins);
+        }
         // 64-bit keys: 8192-key partitions from 1M keys on (digit runs of about 32 keys leave as
         // whole 128-byte lines), 4096-key partitions below, so small sorts still spread over the
         // CUs
@@ -914,6 +1057,35 @@ int run_sort_and_bin(const RasterInputs& in, DeviceScratch& sc, hipStream_t stre
             int32_t* iout = last ? ids_final : sc.gids[dst];
             const int shift = ps.shift[pass];
             const int64_t nb2 = pass == 0 ? 2 * nbins : 0;
+            if (small) {
+                // as below, one launch: kind 0, 1 or 2 of packed keys, or 64-bit keys
+                const int kind = wide ? 3 : !narrow || pass == 0 ? 0 : pass == 1 ? 1 : 2;
+                const int low = kind == 2 ? 16 : 0;  // 16-bit halves count their bits from 16
+                const uint32_t* counts = sc.part_counts + pass * pass_words;
+                uint32_t* next = last ? nullptr : sc.part_counts + (pass + 1) * pass_words;
+                const int next_shift = last ? 0 : ps.shift[pass + 1] - low;
+                const dim3 grid((unsigned)small_parts);
+                void* const ki = wide ? (void*)sc.wkeys[src] : (void*)sc.keys[src];
+                void* const ko = wide ? (void*)sc.wkeys[dst] : (void*)sc.keys[dst];
+                auto go = [&](auto kernel, auto* in, auto* out_keys) {
+                    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, in, vin, sc.gids[src],
+                                       out_keys, vout, iout, M, m_dev, shift - low, counts, next,
+                                       next_shift);
+                };
+                if (kind == 0)
+                    go(small_scatter_kernel<uint32_t, uint32_t>, static_cast<const uint32_t*>(ki),
+                       static_cast<uint32_t*>(ko));
+                else if (kind == 1)
+                    go(small_scatter_kernel<uint32_t, uint16_t>, static_cast<const uint32_t*>(ki),
+                       static_cast<uint16_t*>(ko));
+                else if (kind == 2)
+                    go(small_scatter_kernel<uint16_t, uint16_t>, static_cast<const uint16_t*>(ki),
+                       static_cast<uint16_t*>(ko));
+                else
+                    go(small_scatter_kernel<uint64_t, uint64_t>, static_cast<const uint64_t*>(ki),
+                       static_cast<uint64_t*>(ko));
+                continue;
+            }
             if (wide) {
                 const uint64_t* ki = sc.wkeys[src];
                 uint64_t* ko = sc.wkeys[dst];

@@ -79,7 +79,9 @@ void set_force_wide_keys(bool force);
 
 // Digit passes of the sort: at most 8 bytes of a 64-bit key.
 constexpr int kMaxPasses = 8;
-constexpr int kSortTileMin = 4096;   // keys per radix-sort partition (smallest size used)
+constexpr int kSortTileMin = 4096;   // keys per radix-sort partition (smallest size but the small sort's)
+constexpr int kSortSmallTile = 1024;  // keys per partition of the small sort
+constexpr int64_t kSortSmallM = 80 * kSortSmallTile;  // most keys (or list capacity) it takes
 constexpr int64_t kSortBigM = 1 << 20;  // from this many keys on, partitions hold 8192 keys
 
 // Inputs of sort_and_bin and the blends.
@@ -229,7 +231,7 @@ int launch_project_fwd(const ProjectArgs& a, DeviceScratch& sc, hipStream_t stre
 int launch_project_fwd_into(const ProjectArgs& a, uint32_t* chunk_sums, hipStream_t stream);
 // The fused render forward's projection: also each item's packed blend record (recs, 4 float4
 // per item, from colors / compensate as launch_pack_records would write it) and, with depth_mm
-// non-null (requires n >= 1024), the per-image depth range of the visible items (mm_partial:
+// non-null (requires n >= project_fwd_chunk_items), the per-image depth range of the visible items (mm_partial:
 // scratch of 4 uint32 per chunk), as the sort's depth-range kernels would compute it.
 struct FusedRecords {
     const float* colors; int64_t rows_colors;
@@ -250,10 +252,11 @@ int launch_project_fwd_fused(const ProjectArgs& a, const FusedRecords& f, Device
                              hipStream_t stream);
 int launch_project_fwd_impl(const ProjectArgs& a, uint32_t* chunk_sums, const FusedRecords* f,
                             hipStream_t stream);
-// Items per chunk of the projection's tile-count scan (one projection workgroup each).
-constexpr int64_t kProjChunkItems = 1024;
+// Items per chunk of the projection's tile-count scan over `total` items (one projection workgroup
+// each, 256 or 1024 items), and the number of chunks.
+int32_t project_fwd_chunk_items(int64_t total);
 int64_t project_fwd_chunks(int64_t total);
-// Adds chunk c's exclusive prefix to the items of chunk c (1024 items per chunk), c >= 1.
+// Adds chunk c's exclusive prefix to the items of chunk c, c >= 1.
 int launch_chunk_offsets(int32_t* cum, int64_t total, const uint32_t* chunk_prefix,
                          hipStream_t stream);
 // The projection with no allocation: its chunk totals in a fixed device array of
