@@ -92,154 +92,114 @@ __global__ void __launch_bounds__(256) pack_records_kernel(PackParams P) {
     for (int k = threadIdx.x; k < count; k += 256) dst[k] = s_rec[k];
 }
 
-// Whether a packed record can reach a pixel centre of the 8x8 quadrant whose first one is
-// (qx, qy): its box of half-widths (ex, ey) against the quadrant's. The backward's test: cheaper
-// than the forward's per-band one, and a record that reaches no pixel costs it only the sigma
-// test.
-__device__ __forceinline__ bool box_reaches(const float4& r0, const float4& r3, float qx,
-                                            float qy) {
-    const uint32_t mode = __float_as_uint(r3.z);
-    const bool box = r0.x + r3.x >= qx && r0.x - r3.x <= qx + 7.0f && r0.y + r3.y >= qy &&
-                     r0.y - r3.y <= qy + 7.0f;
-    return mode == kCullBox ? box : mode == kCullKeep;
-}
-
-// The forward's sub-block mask: the sub-blocks whose pixel centres the record can reach, from the
-// exact x-extent of its ellipse over each 4-row band of the tile's pixel centres (the box test
-// above also keeps sub-blocks that only the box's corners reach; on config 2 the forward's row
-// walks take 23% fewer steps with this mask).
+// The 16 sub-blocks of tile (tile_x, tile_y) whose pixel centres the record can reach, bit 4 j + i
+// for sub-block i of band j, from the exact x-extent of its ellipse over each 4-row band of the
+// tile's pixel centres (a box test would also keep the sub-blocks that only the box's corners
+// reach: 23% more steps of the forward's row walks at 1M gaussians, 1920x1080).
 // With Q(dx, dy) = a/2 dx^2 + b dx dy + c/2 dy^2 (dx, dy from the centre), the test uses the
 // ellipse Q <= s' with s' = 1.0201 sigma_max, i.e. {sigma <= sigma_max} scaled by 1.01: an
-// evaluated sigma <= sigma_max has an exact Q within 0.6% of it for the conics the box mode
-// accepts ((a + c)^2 / det < 1e4), so every such pixel centre lies inside. The chord of that
-// ellipse at height dy is centred at -b dy / a with half-width sqrt(2 a s' - det dy^2) / a, so its
-// right end is concave in dy and peaks at the rightmost point (dx, dy) = (ex, -b ex / c), ex =
-// sqrt(2 s' c / det); over a band [dy0, dy1] clipped to |dy| <= ey the extent is therefore
-// [min of the left ends at dy0 and dy1, or -ex when the leftmost point lies in the band,
-//  max of the right ends, or ex when the rightmost point lies in it], widened by m = 0.01 px +
-// 1e-3 ex against rounding (the rows are clipped to |dy| <= ey + m, where the chord's width is
-// taken as 0 beyond ey). A sub-block is kept when its pixel-centre columns meet that extent.
+// evaluated sigma <= sigma_max has an exact Q within 0.6% of it for the conics the record keeps a
+// chord for ((a + c)^2 / det < 1e4), so every such pixel centre lies inside, with more than 1% of
+// s' left for the rounding of det (at most 3e-4 of it there). The chord at height dy runs from
+// s dy - W to s dy + W with s = -b / a, W = sqrt(P - D dy^2), P = 2 s' / a, D = det / a^2. Its
+// right end is concave in dy with its peak at dy_r, so over the band [y0, y1] it is largest at
+// dy_r clamped to the band, and the left end is smallest at -dy_r clamped. Both are widened by
+// m = 0.01 px + 1e-3 of the ellipse's half-width against rounding. A band that misses the ellipse
+// has P - D dy^2 < 0 at both heights: the NaN of the square root keeps no sub-block.
+// All lengths along x are in sub-blocks (s, W, m / 4; P, D / 16), so the counts of sub-blocks from
+// the tile's left edge to the right end, and from its right edge to the left end, are the
+// truncations below; a record without a trusted chord has m = 1e30 and P = D = 0 (all
+// sub-blocks), one that no pixel accepts P < 0 or NaN. 21 VALU and two square roots per band: the
+// chords at both ends of the band with a select for the peak, then a compare per sub-block, took
+// 221 VALU per record where this takes about 100.
 constexpr float kTightScale2 = 1.0201f;
-
-// The tile-relative quantities of that test for one kCullBox record. The record carries the
-// tile-independent parts, formed once per item by the pack: 1 / a in r1.w, the scaled ellipse's
-// half-widths as the box's minus its 0.01 px, and the rightmost point's height in r3.w.
-struct TightEllipse {
-    float det, inv_a, ex, ey, dy_r, m, two_a_s, nb_a, bx, by;
-};
-__device__ __forceinline__ TightEllipse tight_setup(const float4& r0, const float4& r1,
-                                                    const float4& r3, int tile_x, int tile_y) {
-    TightEllipse e;
-    const float a = 2.0f * r0.z, b = r0.w, c = 2.0f * r1.x;
-    const float s2 = 2.0f * (kTightScale2 * r1.z);  // 2 s'
-    e.det = a * c - b * b;
-    e.inv_a = r1.w;
-    e.ex = r3.x - 0.01f;
-    e.ey = r3.y - 0.01f;
-    e.dy_r = r3.w;  // rightmost point; leftmost at -dy_r
-    e.m = 0.01f + 1e-3f * e.ex;
-    e.two_a_s = a * s2;
-    e.nb_a = -b * e.inv_a;
-    e.bx = (float)(tile_x * kBlockWidth) + 0.5f - r0.x;  // dx of the tile's first column
-    e.by = (float)(tile_y * kBlockWidth) + 0.5f - r0.y;
-    return e;
-}
-
-// Bits 4 j .. 4 j + 3 of the mask: the sub-blocks of band j (pixel-centre rows 4 j .. 4 j + 3).
-__device__ __forceinline__ uint32_t tight_band(const TightEllipse& e, int j) {
-    const float y0 = e.by + (float)(4 * j);
-    const float d0 = fmaxf(y0, -e.ey - e.m), d1 = fminf(y0 + 3.0f, e.ey + e.m);
-    const float w0 = __builtin_amdgcn_sqrtf(fmaxf(e.two_a_s - e.det * (d0 * d0), 0.0f)) * e.inv_a;
-    const float w1 = __builtin_amdgcn_sqrtf(fmaxf(e.two_a_s - e.det * (d1 * d1), 0.0f)) * e.inv_a;
-    const float c0 = e.nb_a * d0, c1 = e.nb_a * d1;
-    float hi = fmaxf(c0 + w0, c1 + w1), lo = fminf(c0 - w0, c1 - w1);
-    hi = (e.dy_r >= d0 && e.dy_r <= d1) ? e.ex : hi;
-    lo = (-e.dy_r >= d0 && -e.dy_r <= d1) ? -e.ex : lo;
-    hi = hi + e.m;
-    lo = lo - e.m;
-    const bool band = d0 <= d1;  // the band's rows meet |dy| <= ey + m
-    uint32_t bits = 0u;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float x0 = e.bx + (float)(4 * i);
-        bits |= (band && x0 <= hi && x0 + 3.0f >= lo) ? (1u << (4 * j + i)) : 0u;
-    }
-    return bits;
-}
-
-__device__ __forceinline__ uint32_t subblock_mask_tight(const float4& r0, const float4& r1,
-                                                        const float4& r3, int tile_x,
-                                                        int tile_y) {
-    const uint32_t mode = __float_as_uint(r3.z);
-    if (mode == kCullNone) return 0u;
-    if (mode != kCullBox) return 0xffffu;
-    const TightEllipse e = tight_setup(r0, r1, r3, tile_x, tile_y);
+__device__ __forceinline__ uint32_t subblock_mask(const float4& r0, const float4& r1,
+                                                  const float4& r3, int tile_x, int tile_y) {
+    const float m = r3.x, d = r3.y, dy_r = r3.w;
+    const float p = (0.5f * kTightScale2) * r1.z * r1.w, s = -r0.w * r1.w;
+    const float bx = ((float)(tile_x * kBlockWidth) + 0.5f) - r0.x;  // dx of the first column
+    const float by = ((float)(tile_y * kBlockWidth) + 0.5f) - r0.y;
+    const float k_right = fmaf(bx, -0.25f, m + 1.0f), k_left = fmaf(bx, 0.25f, m + 4.75f);
     uint32_t mask = 0u;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) mask |= tight_band(e, j);
+    for (int j = 0; j < 4; ++j) {
+        const float y0 = by + (float)(4 * j), y1 = by + (float)(4 * j + 3);
+        const float tr = __builtin_amdgcn_fmed3f(dy_r, y0, y1);
+        const float tl = __builtin_amdgcn_fmed3f(-dy_r, y0, y1);
+        const float wr = __builtin_amdgcn_sqrtf(fmaf(-(d * tr), tr, p));
+        const float wl = __builtin_amdgcn_sqrtf(fmaf(-(d * tl), tl, p));
+        const float hr = fmaf(s, tr, wr + k_right), hl = fmaf(-s, tl, wl + k_left);
+        const uint32_t nr = (uint32_t)__builtin_amdgcn_fmed3f(hr, 0.0f, 4.0f);
+        const uint32_t nl = (uint32_t)__builtin_amdgcn_fmed3f(hl, 0.0f, 4.0f);
+        const uint32_t width = __builtin_elementwise_sub_sat(nr + nl, 4u);
+        mask |= ((1u << width) - 1u) << ((uint32_t)(4 * j + 4) - nl);
+    }
     return mask;
 }
 
-// LDS records of one batch: r0 = (x, y, a/2, b), r1 = (c/2, o, sigma_max, 1/a), r2 = (red, green,
-// blue, depth), each record's sub-block mask, and one compacted record list per sub-block, of
-// record byte offsets (16 t for slot t: the address needs no shift).
+// LDS records of one batch: r0 = (x, y, a/2, b), r1 = (c/2, o, sigma_max, mask), r2 = (red, green,
+// blue, depth), and one compacted record list per sub-block, of record byte offsets (16 t for slot
+// t: the address needs no shift). mask (bits, in the place of the record's 1/(4a)) is the record's
+// sub-block mask, with kMaskClamped where its opacity exceeds kAlphaMax.
 template <int kBatch>
 struct BatchLds {
     float4 r0[kBatch];
     float4 r1[kBatch];
     float4 r2[kBatch];
-    uint16_t mask[kBatch];
     __attribute__((aligned(8))) uint16_t list[16][kBatch];
 };
+constexpr uint32_t kMaskClamped = 1u << 16;
 
 // Stages the record of item `id` (the sorted range's entry for slot `tid`) into slot `tid` (one
 // barrier), then each wave builds the lists of its four sub-blocks (one per 16-lane row) from the
 // staged masks, in slot order; row r leaves out the slots below first[r]. `live` is false for the
 // clamped tail slots of the last batch (they reach no sub-block). Returns the length of the
-// wave's longest list plus 65536 times the calling lane's row list length.
+// wave's longest list plus 65536 times the calling lane's row list length; `clamped` tells whether
+// an opacity of the batch exceeds kAlphaMax.
 template <int kBatch, bool kFirst>
 __device__ __forceinline__ int stage_batch(const BlendCommon& C, BatchLds<kBatch>& L, int32_t id,
                                            bool live, int tile_x, int tile_y,
-                                           const int (&first)[4], int32_t* s_clamped) {
+                                           const int (&first)[4], bool& clamped) {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, row = lane >> 4;
     int64_t g = id;
     if (kBatch == kTile || tid < kBatch) {
-        uint32_t m = 0u;
         float4 r0 = make_float4(0.f, 0.f, 0.f, 0.f), r1 = r0, r2 = r0;
         if (live && g >= 0 && g < C.total) {
             const float4* rec = C.recs + 4 * g;
             r0 = rec[0];
             r1 = rec[1];
             r2 = rec[2];
-            m = subblock_mask_tight(r0, r1, rec[3], tile_x, tile_y);
+            uint32_t m = subblock_mask(r0, r1, rec[3], tile_x, tile_y);
+            if (r1.y > kAlphaMax) m |= kMaskClamped;
+            r1.w = __uint_as_float(m);
         }
         L.r0[tid] = r0;
         L.r1[tid] = r1;
         L.r2[tid] = r2;
-        L.mask[tid] = (uint16_t)m;
-        if constexpr (kFirst) {
-            const bool any = __ballot(r1.y > kAlphaMax) != 0ull;
-            if (lane == 0) s_clamped[wave] = any;
-        }
     }
     __syncthreads();
     // this wave's sub-blocks: rows 0..3 -> sb0, sb0 + 1, sb0 + 4, sb0 + 5
     const int sb0 = (wave >> 1) * 8 + (wave & 1) * 2;
-    const uint64_t lt = (1ull << lane) - 1ull;
     int n[4] = {0, 0, 0, 0};
+    uint32_t any = 0u;
 #pragma unroll
     for (int c = 0; c < (kBatch + 63) / 64; ++c) {
         const int slot = c * 64 + lane;
-        const uint32_t mc = (kBatch % 64 == 0 || slot < kBatch) ? L.mask[slot] : 0u;
+        const uint32_t mc =
+            (kBatch % 64 == 0 || slot < kBatch) ? __float_as_uint(L.r1[slot].w) : 0u;
+        any |= mc;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int b = sb0 + (r & 1) + (r >> 1) * 4;
             const bool bit = ((mc >> b) & 1u) && (!kFirst || slot >= first[r]);
             const uint64_t bal = __ballot(bit);
-            if (bit) L.list[b][n[r] + (int)__popcll(bal & lt)] = (uint16_t)(slot * 16);
+            const int before = (int)__builtin_amdgcn_mbcnt_hi(
+                (uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+            if (bit) L.list[b][n[r] + before] = (uint16_t)(slot * 16);
             n[r] += (int)__popcll(bal);
         }
     }
+    clamped = __ballot((any & kMaskClamped) != 0u) != 0ull;
     __builtin_amdgcn_wave_barrier();
     const int mine = row == 0 ? n[0] : row == 1 ? n[1] : row == 2 ? n[2] : n[3];
     const int a = n[0] > n[1] ? n[0] : n[1], b = n[2] > n[3] ? n[2] : n[3];
@@ -288,7 +248,7 @@ __device__ __forceinline__ float blend_sigma(const float4& r0, const float4& r1,
 
 // 0 <= sigma <= sigma_max as one unsigned compare of the float bits (one VALU where two float
 // compares take two). Equal for every record a list holds: its sigma_max is >= 0 and not NaN
-// (a record with sigma_max < 0 or NaN is kCullNone and reaches no sub-block); sigma is never
+// (a record with sigma_max < 0 or NaN reaches no sub-block); sigma is never
 // -0.0 (with c > 0 the term (c/2 dy) dy is +0 or positive, and a rounded sum is -0.0 only when
 // both addends are), so a negative sigma has its sign bit set and fails, as a NaN does.
 __device__ __forceinline__ bool sigma_in_range(float sigma, float sigma_max) {
@@ -309,10 +269,15 @@ struct BlendFwdParams {
 
 // kDepth adds the expected-depth channel of _rasterize_depth_kernel
 // (splax/_rasterize/_kernels.py:277-383): depth times the same blend weight, no background term.
-// At most 72 VGPRs: seven waves per SIMD (0.187 ms at config 2 against 0.195 at the compiler's
-// own 79 VGPRs and six; forcing eight spills registers).
+// Bound by VALU issue, and by what the scalar unit and the branches add where a step's VALU do not
+// cover them. At most 64 VGPRs and 20480 bytes of LDS (no array beside the batch's: masks, wave
+// flags and loss sums take places that are free at the time), so eight waves per SIMD. At 1M
+// gaussians, 1920x1080: 163 us (153 with depth), at 8 views of 200K 430 us. Before: seven waves, a
+// workgroup-wide count of done pixels per batch (three barriers), masks of 221 VALU, a flag for a
+// done pixel and both loop bounds in every step: 189, 189 and 498 us. The cheaper masks and the
+// one barrier alone were 181 with depth and 489 us, and the rest is the shorter step.
 template <bool kDepth>
-__global__ void __launch_bounds__(kTile, 7) blend_fwd_kernel(BlendFwdParams P) {
+__global__ void __launch_bounds__(kTile, 8) blend_fwd_kernel(BlendFwdParams P) {
     __shared__ BatchLds<kTile> L;
     const BlendCommon& C = P.c;
     const int tid = threadIdx.x;
@@ -339,53 +304,69 @@ __global__ void __launch_bounds__(kTile, 7) blend_fwd_kernel(BlendFwdParams P) {
     const char* rec_base = reinterpret_cast<const char*>(L.r0);
 
     for (int32_t bt = 0; bt < num_batches; ++bt) {
-        // every pixel done -> stop; also the barrier before the LDS records are overwritten
-        if (__syncthreads_count(done) >= kTile) break;
+        // every pixel done -> stop; also the barrier before the LDS records are overwritten. Each
+        // wave's flag takes the place of the first entry of its own first list, which no walk
+        // reads by now and which is built anew after stage_batch's barrier.
+        const uint64_t live = __ballot(!done);
+        if ((tid & 63) == 0) L.list[sb][0] = live != 0ull;
+        __syncthreads();
+        if (!(L.list[0][0] | L.list[2][0] | L.list[8][0] | L.list[10][0])) break;
         const int32_t batch_start = range_start + bt * kTile;
         const int32_t src = iminw(batch_start + tid, range_end - 1);
+        bool clamped;
         const int lens = stage_batch<kTile, false>(C, L, C.ids[src],
                                                    batch_start + tid < range_end, tile_x, tile_y,
-                                                   {0, 0, 0, 0}, nullptr);
-        if (__ballot(!done) == 0ull) continue;
-        const int wave_max = lens & 0xffff, my_len = lens >> 16;  // my_len uniform per row
+                                                   {0, 0, 0, 0}, clamped);
+        if (live == 0ull) continue;
+        int len = done ? -1 : lens >> 16;
         const uint16_t* list = L.list[sb];
         int32_t last_off = -1;  // the last accepted record of this batch (byte offset)
-        for (int k = 0; k < wave_max; ++k) {
-            // A lane leaves once its pixel is done or its row's list is walked; the wave walks
-            // while any lane is left, which is exec-mask bookkeeping only. (Padding the shorter
-            // lists with a record no pixel accepts instead of the length test measured slower.)
-            if (done || k >= my_len) break;
-            const int off = list[k];
-            const float4 r0 = *reinterpret_cast<const float4*>(rec_base + off);
-            const float4 r1 = *reinterpret_cast<const float4*>(rec_base + off + sizeof(L.r0));
-            // all of r1 in the first read (one full-width read, one address)
-            asm volatile("" ::"v"(r1.y));
-            const float dx = r0.x - px, dy = r0.y - py;
-            const float sigma = blend_sigma(r0, r1, dx, dy);
-            // Nested conditions and the one exit above: every other path falls through to the
-            // next step, which keeps the loop's control flow in the exec mask.
-            if (sigma_in_range(sigma, r1.z)) {
-                // v_min: no accepted record has a NaN opacity (the pack culls those), so it
-                // equals the reference's compare-and-select minimum here
-                const float alpha = fminf(kAlphaMax, r1.y * blend_exp(-sigma, exp_round, exp_c5));
-                if (alpha >= kAlphaThresh) {
-                    const float next_T = T * (1.0f - alpha);
-                    if (next_T <= kTEps) {
-                        done = true;  // leaves at the next step
-                    } else {
-                        const float4 r2 = *reinterpret_cast<const float4*>(
-                            rec_base + off + 2 * sizeof(L.r0));
-                        const float vis = alpha * T;
-                        o0 = fmaf(r2.x, vis, o0);
-                        o1 = fmaf(r2.y, vis, o1);
-                        o2 = fmaf(r2.z, vis, o2);
-                        if constexpr (kDepth) od = fmaf(r2.w, vis, od);
-                        T = next_T;
-                        last_off = off;
+        auto walk = [&](auto clamp) {
+            // A lane leaves once its row's list is walked or its pixel is done (len = -1); the wave
+            // walks while any lane is left, which is exec-mask bookkeeping only. (Padding the
+            // shorter lists with a record no pixel accepts instead of the length test measured
+            // slower; a separate flag for a done pixel costs up to six VALU per step.)
+            for (int k = 0; k < len; ++k) {
+                const int off = list[k];
+                const float4 r0 = *reinterpret_cast<const float4*>(rec_base + off);
+                const float4 r1 = *reinterpret_cast<const float4*>(rec_base + off + sizeof(L.r0));
+                // all of r1 in the first read (one full-width read, one address)
+                asm volatile("" ::"v"(r1.y));
+                const float dx = r0.x - px, dy = r0.y - py;
+                const float sigma = blend_sigma(r0, r1, dx, dy);
+                // Nested conditions and the one exit above: every other path falls through to the
+                // next step, which keeps the loop's control flow in the exec mask.
+                if (sigma_in_range(sigma, r1.z)) {
+                    // v_min: no accepted record has a NaN opacity (the pack culls those), so it
+                    // equals the reference's compare-and-select minimum here
+                    float alpha = r1.y * blend_exp(-sigma, exp_round, exp_c5);
+                    if constexpr (decltype(clamp)::value) alpha = fminf(kAlphaMax, alpha);
+                    if (alpha >= kAlphaThresh) {
+                        const float next_T = T * (1.0f - alpha);
+                        const bool stop = next_T <= kTEps;
+                        len = stop ? -1 : len;  // leaves at the next step
+                        asm("" : "+v"(len));  // one select here, not moves on three paths
+                        if (!stop) {
+                            const float4 r2 = *reinterpret_cast<const float4*>(
+                                rec_base + off + 2 * sizeof(L.r0));
+                            const float vis = alpha * T;
+                            o0 = fmaf(r2.x, vis, o0);
+                            o1 = fmaf(r2.y, vis, o1);
+                            o2 = fmaf(r2.z, vis, o2);
+                            if constexpr (kDepth) od = fmaf(r2.w, vis, od);
+                            T = next_T;
+                            last_off = off;
+                        }
                     }
                 }
             }
-        }
+        };
+        // without a record opaque enough for its alpha to be clamped a step takes one VALU less
+        if (clamped)
+            walk(std::true_type{});
+        else
+            walk(std::false_type{});
+        done = len < 0;
         if (last_off >= 0) cur_idx = batch_start + (last_off >> 4);
     }
     double err = 0.0;  // this pixel's part of the fused loss
@@ -411,12 +392,19 @@ __global__ void __launch_bounds__(kTile, 7) blend_fwd_kernel(BlendFwdParams P) {
         }
     }
     if (P.loss_kind != kLossNone) {  // uniform; every lane active again for the DPP sum
-        __shared__ double s_err[kTile / 64];
+        // each wave's sum in its own second list: another wave may still be walking its lists, or
+        // reading the flags in the first ones
         err = wave_sum_f64_to_lane63(err);
-        if ((tid & 63) == 63) s_err[tid >> 6] = err;
+        if ((tid & 63) == 63) __builtin_memcpy(L.list[sb - 4], &err, sizeof(err));
         __syncthreads();
-        if (tid == 0)
-            P.loss_partials[tile_g] = ((s_err[0] + s_err[1]) + s_err[2]) + s_err[3];
+        if (tid == 0) {
+            double e[4];
+            __builtin_memcpy(&e[0], L.list[1], 8);
+            __builtin_memcpy(&e[1], L.list[3], 8);
+            __builtin_memcpy(&e[2], L.list[9], 8);
+            __builtin_memcpy(&e[3], L.list[11], 8);
+            P.loss_partials[tile_g] = ((e[0] + e[1]) + e[2]) + e[3];
+        }
     }
 }
 
@@ -731,7 +719,7 @@ __global__ void __launch_bounds__(kTile, kDepth ? 5 : 6) blend_bwd_kernel(BlendB
     constexpr int NG = kDepth ? 10 : 9;
     __shared__ BatchLds<kBwdBatch> L;
     __shared__ float acc[4][NG][kBwdStride];
-    __shared__ int32_t s_max, s_clamped[2];
+    __shared__ int32_t s_max;
 
     const BlendCommon& C = P.c;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -863,9 +851,9 @@ __global__ void __launch_bounds__(kTile, kDepth ? 5 : 6) blend_bwd_kernel(BlendB
         }
         const int first[4] = {batch_end - rmax[0], batch_end - rmax[1], batch_end - rmax[2],
                               batch_end - rmax[3]};
+        bool clamped;
         const int lens = stage_batch<kBwdBatch, true>(C, L, id, live, tile_x, tile_y, first,
-                                                      s_clamped);
-        const bool clamped = uniform(s_clamped[0] | s_clamped[1]) != 0;
+                                                      clamped);
         const int wave_max = uniform(lens & 0xffff), my_len = lens >> 16;  // uniform per row
         const uint16_t* const list = L.list[sb];
         const int32_t min_off = (batch_end - bin_final) * 16;  // the pixel's first record

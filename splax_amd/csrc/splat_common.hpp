@@ -415,14 +415,15 @@ __device__ __forceinline__ float lane63(float v) {
 constexpr float kBlendSigmaCap = 87.0f;
 
 // Packed record of one geometry item, 64 bytes (one aligned segment per staged intersection):
-//   r0 = (x, y, a/2, b), r1 = (c/2, o, sigma_max, 1/a), r2 = (red, green, blue, depth),
-//   r3 = (ex, ey, cull mode, dy_r) (1/a and dy_r, the height of the 1.01-scaled ellipse's
-//   rightmost point, for the forward's tight sub-block test; 0 unless the cull mode is the box).
+//   r0 = (x, y, a/2, b), r1 = (c/2, o, sigma_max, 1/(4a)), r2 = (red, green, blue, depth),
+//   r3 = (m, D, cull mode, dy_r).
 // They depend only on the rasterizer's inputs, so a forward's records serve its backward.
-// sigma_max = log(255 o) + 1e-3 bounds sigma where o e^-sigma can still reach 1/255. The cull mode
-// says whether the tile-independent box (+-ex, +-ey) around the centre holds every pixel centre
-// with sigma <= sigma_max (kCullBox), or no pixel can pass (kCullNone: sigma_max < 0), or the box
-// cannot be trusted and every quadrant is kept (kCullKeep).
+// sigma_max = log(255 o) + 1e-3 bounds sigma where o e^-sigma can still reach 1/255. 1/(4a), D, dy_r
+// and m give the chords of the ellipse {sigma <= sigma_max} scaled by 1.01, for the blends'
+// sub-block masks (subblock_mask). The cull mode says whether they hold every pixel centre with
+// sigma <= sigma_max (kCullBox), or no pixel can pass (kCullNone: sigma_max < 0 or NaN), or the
+// chords cannot be trusted and every sub-block is kept (kCullKeep); the fields alone give the same
+// masks.
 enum : uint32_t { kCullBox = 0u, kCullKeep = 1u, kCullNone = 2u };
 
 // The record of one item from its projection outputs (xy, conic a b c, depth), its raw opacity
@@ -444,37 +445,37 @@ __device__ __forceinline__ void pack_record(float x, float y, float a, float b, 
         smax = -__builtin_inff();  // o <= 0 or NaN: no pixel accepts it
     }
     uint32_t mode = kCullKeep;
-    float ex = 0.0f, ey = 0.0f, inv_a = 0.0f, dy_r = 0.0f;
+    float ia4 = 0.0f, m = 1e30f, d = 0.0f, dy_r = 0.0f;
     if (!(smax >= 0.0f)) {
         mode = kCullNone;  // every pixel rejected
+        ia4 = 1.0f;
+        m = 0.0f;
     } else {
         // Points beyond k times the bounding box of {sigma <= smax} have exact
         // sigma >= k^2 smax. The evaluated sigma differs from the exact one by at most
         // ~6e-7 * cond(Q) relative (Q the conic), so with cond(Q) <= (a + c)^2 / det < 1e4
-        // and k = 1.01 every point outside the box evaluates above smax.
-        // Worse-conditioned conics keep all four quadrants.
+        // and k = 1.01 every point outside the scaled ellipse evaluates above smax.
+        // Worse-conditioned conics keep all sub-blocks. The margins are orders of magnitude above
+        // the error of the hardware's reciprocal and square root (1 ulp each); one det serves all
+        // fields, so P - D dy_r^2 stays positive where det / (a c) is small.
         const float det = a * c - b * b;
         const float tr = a + c;
-        const float ex2 = 2.0f * smax * c / det, ey2 = 2.0f * smax * a / det;
-        if (a > 0.0f && c > 0.0f && det > 0.0f && tr * tr < 1e4f * det && ex2 < 1e30f &&
-            ey2 < 1e30f) {
-            // half-widths of the ellipse {sigma <= 1.0201 smax} (the 1.01-scaled one), and the box
-            const float sx = sqrtf(ex2) * 1.01f, sy = sqrtf(ey2) * 1.01f;
-            ex = sx + 0.01f;
-            ey = sy + 0.01f;
-            // for the forward's tight sub-block test: 1 / a and the height of the scaled
-            // ellipse's rightmost point relative to its centre
-            inv_a = 1.0f / a;
-            dy_r = -(b * sx) / c;
+        const float k = 2.0f * smax * __builtin_amdgcn_rcpf(det);
+        if (a > 0.0f && c > 0.0f && det > 0.0f && tr * tr < 1e4f * det && k * tr < 1e30f) {
+            const float ex = __builtin_amdgcn_sqrtf(k * c) * 1.01f;  // the half-width
+            ia4 = 0.25f * __builtin_amdgcn_rcpf(a);
+            m = fmaf(2.5e-4f, ex, 2.5e-3f);
+            d = (det * ia4) * ia4;
+            dy_r = -(b * ex) * __builtin_amdgcn_rcpf(c);
             mode = kCullBox;
         }
     }
     // the blends evaluate sigma = (a/2 dx dx + c/2 dy dy) + b dx dy: halving exactly before
     // the products leaves every rounding where 0.5 (a dx dx + c dy dy) puts it
     r[0] = make_float4(x, y, 0.5f * a, b);
-    r[1] = make_float4(0.5f * c, o, smax, inv_a);
+    r[1] = make_float4(0.5f * c, o, smax, ia4);
     r[2] = make_float4(color[0], color[1], color[2], depth);
-    r[3] = make_float4(ex, ey, __uint_as_float(mode), dy_r);
+    r[3] = make_float4(m, d, __uint_as_float(mode), dy_r);
 }
 
 }  // namespace splat
