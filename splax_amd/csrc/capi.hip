@@ -599,9 +599,9 @@ int splat_project_fwd_noalloc(splat_stream_t stream, const float* means3d, int64
                               clip_thresh, xys, depths, radii, conics, num_tiles_hit,
                               cum_tiles_hit, quats_wxyz, &a);
     if (rc) return rc;
-    if (project_fwd_chunks(total) > kNoAllocMaxChunks)
+    if (total > kNoAllocMaxItems)
         return fail(kErrArgs, "project_fwd_noalloc: more than " +
-                                  std::to_string(kNoAllocMaxChunks * 1024) +
+                                  std::to_string(kNoAllocMaxItems) +
                                   " items (the size of its fixed scratch)");
     // no library scratch, stage timer or stream bookkeeping: nothing here allocates
     g_last_error.clear();
@@ -1193,7 +1193,7 @@ int splat_render_fwd(splat_stream_t stream, const float* means3d, int64_t rows_m
     if (L.overflow) return fail(kErrKeyOverflow, "render_fwd: intersection key overflow");
     sc.workload(B, num_gaussians, L.num_tiles);
     // the depth range from the projection: packed key, chunks meeting at most two images
-    const bool fuse_range = L.packed && num_gaussians >= project_fwd_chunk_items(total);
+    const bool fuse_range = L.packed && num_gaussians >= kProjChunk;
     const int64_t chunks = project_fwd_chunks(total);
     {
         const int32_t bpi = (num_gaussians + 4095) / 4096;

@@ -33,6 +33,8 @@ struct ProjectParams {
     int64_t total;
     int32_t img_h, img_w;
     float fx, fy, cx, cy, glob_scale, clip_thresh;
+    float lim_x, lim_y;  // kFovClamp times the half field of view's tangents
+    ItemDiv by_n;
     float* xys; float* depths; int32_t* radii; float* conics;
     int32_t* num_tiles_hit; int32_t* cum_tiles_hit;
     int32_t wxyz;  // quaternion storage order: 1 = wxyz (the public API's), 0 = xyzw
@@ -46,17 +48,6 @@ struct ProjectParams {
 };
 
 constexpr int kProjThreads = 256;
-// Items per chunk of the projection's tile-count scan (one forward workgroup each, one item per
-// thread): 1024 keeps the chunk-total scan short (about 12 totals per scan thread at 12M items).
-// Up to kProjSmallItems items the chunks hold 256: with 1024 they would be fewer than the CUs, and
-// the projection is bound by VALU issue on the CUs it runs on (10K items are 10 workgroups of
-// 1024, 10.0 us, or 40 of 256, 6.5 us; 100K items 13.9 and 11.7 us).
-constexpr int kProjChunkBig = 1024, kProjChunkSmall = 256;
-constexpr int64_t kProjSmallItems = 256 * kProjChunkBig;
-int32_t project_fwd_chunk_items(int64_t total) {
-    return total <= kProjSmallItems ? kProjChunkSmall : kProjChunkBig;
-}
-
 __device__ __forceinline__ bool apply_transform(const float* transforms, int32_t image_id,
                                                 int32_t num_transforms, bool sel_tf,
                                                 int32_t tf_id, float* mean, float* R_tf) {
@@ -120,9 +111,9 @@ struct ItemOut {
 };
 
 // Per-item projection; writes the item's outputs and returns them (count 0 when culled).
-__device__ __forceinline__ ItemOut project_item(const ProjectParams& P, int64_t idx) {
+__device__ __forceinline__ ItemOut project_item(const ProjectParams& P, int64_t idx, int32_t bid) {
     const int32_t n = P.n;
-    const int32_t bid = (int32_t)(idx / n), gid = (int32_t)(idx - (int64_t)bid * n);
+    const int32_t gid = (int32_t)(idx - (int64_t)bid * n);
     const int64_t m_idx = P.rows_means > n ? idx : gid;
     const int64_t s_idx = P.rows_scales > n ? idx : gid;
     const int64_t q_idx = P.rows_quats > n ? idx : gid;
@@ -163,14 +154,20 @@ __device__ __forceinline__ ItemOut project_item(const ProjectParams& P, int64_t 
         if (p[2] <= P.clip_thresh) break;
         float V[9];
         mat_mul_nt(M, M, V);
-        const float tan_fovx = 0.5f * (float)P.img_w / P.fx;
-        const float tan_fovy = 0.5f * (float)P.img_h / P.fy;
-        const float lim_x = kFovClamp * tan_fovx;
-        const float lim_y = kFovClamp * tan_fovy;
         float tz = p[2];
-        float tx = tz * minw(lim_x, maxw(-lim_x, p[0] / tz));
-        float ty = tz * minw(lim_y, maxw(-lim_y, p[1] / tz));
-        float rz = 1.0f / tz;
+        const float tw = p[2] + kZEps;
+        const Recip rtz = recip(tz);
+        float px_z = quot(p[0], rtz), py_z = quot(p[1], rtz), rz = quot(1.0f, rtz);
+        float rw = quot(1.0f, recip(tw));
+        if (!(min3_abs(p[0], p[1], tz) >= 0x1p-60f && max3_abs(p[0], p[1], tz) <= 0x1p60f &&
+              tw >= 0x1p-60f && tw <= 0x1p60f)) {
+            px_z = p[0] / tz;
+            py_z = p[1] / tz;
+            rz = 1.0f / tz;
+            rw = 1.0f / tw;
+        }
+        float tx = tz * minw(P.lim_x, maxw(-P.lim_x, px_z));
+        float ty = tz * minw(P.lim_y, maxw(-P.lim_y, py_z));
         float rz2 = rz * rz;
         float j00 = P.fx * rz, j02 = -P.fx * tx * rz2, j11 = P.fy * rz, j12 = -P.fy * ty * rz2;
         float T0[3], T1[3];
@@ -191,16 +188,22 @@ __device__ __forceinline__ ItemOut project_item(const ProjectParams& P, int64_t 
         float cxx = c00 + kDilation, cxy = c01, cyy = c11 + kDilation;
         float det = cxx * cyy - cxy * cxy;
         if (det == 0.0f) break;
-        float inv_det = 1.0f / det;
+        float inv_det = quot(1.0f, recip(det));
+        if (!(__builtin_fabsf(det) >= 0x1p-60f && __builtin_fabsf(det) <= 0x1p60f))
+            inv_det = 1.0f / det;
         float a = cyy * inv_det, b = -cxy * inv_det, c = cxx * inv_det;
-        float rw = 1.0f / (p[2] + kZEps);
         float center_x = (p[0] * rw) * P.fx + P.cx;
         float center_y = (p[1] * rw) * P.fy + P.cy;
         if (opac < kAlphaThresh) break;
         float t = iso_level(opac);
-        float ext = sqrtf(t);
-        float radius_x = ceilf(ext * sqrtf(cxx));
-        float radius_y = ceilf(ext * sqrtf(cyy));
+        float ext = sqrt_mod(t), sx = sqrt_mod(cxx), sy = sqrt_mod(cyy);
+        if (!(min3_abs(t, cxx, cyy) >= kSqrtLo && max3_abs(t, cxx, cyy) <= kSqrtHi)) {
+            ext = sqrtf(t);
+            sx = sqrtf(cxx);
+            sy = sqrtf(cyy);
+        }
+        float radius_x = ceilf(ext * sx);
+        float radius_y = ceilf(ext * sy);
         if (radius_x <= 0.0f && radius_y <= 0.0f) break;
         if (center_x + radius_x <= 0.0f || center_x - radius_x >= (float)P.img_w ||
             center_y + radius_y <= 0.0f || center_y - radius_y >= (float)P.img_h)
@@ -229,13 +232,17 @@ __device__ __forceinline__ ItemOut project_item(const ProjectParams& P, int64_t 
 }
 
 // kFused (the fused render forward): also the item's packed blend record and the chunk's depth
-// range partials (the chunk spans at most two images: num_gaussians >= kThreads). One item per
+// range partials (the chunk spans at most two images: num_gaussians >= kProjChunk). One item per
 // thread keeps the loads coalesced and gives the projection the most waves in flight.
-template <bool kFused, int kThreads>
-__global__ void __launch_bounds__(kThreads) project_fwd_kernel(ProjectParams P) {
+template <bool kFused>
+__global__ void __launch_bounds__(kProjChunk) project_fwd_kernel(ProjectParams P) {
+    constexpr int kThreads = kProjChunk;
     constexpr int kProjItems = 1;
     __shared__ int32_t s_wave[kThreads / 64];
     __shared__ uint32_t s_mm[kThreads / 64][4];
+    // the records of each wave's items, part q of lane l's at 4 l + (q ^ (l >> 2 & 3)): both the
+    // writes and the reads below then take every bank once per 16 lanes
+    __shared__ float4 s_rec[kFused ? kThreads * 4 : 1];
     const int tid = threadIdx.x;
     const uint32_t part = blockIdx.x;
     const int64_t base = (int64_t)part * (kThreads * kProjItems);
@@ -251,22 +258,24 @@ __global__ void __launch_bounds__(kThreads) project_fwd_kernel(ProjectParams P) 
         if (idx < P.total) {
             // the record's colour is loaded with the item's other inputs, not after its stores
             float col[3] = {0.f, 0.f, 0.f};
+            const int32_t bid = (int32_t)item_quot(idx, P.by_n);
             if constexpr (kFused) {
-                const float* cp = P.colors + 3 * (idx % P.rows_colors);
+                const int64_t crow = P.rows_colors == P.n ? idx - (int64_t)bid * P.n
+                                     : P.rows_colors >= P.total ? idx : idx % P.rows_colors;
+                const float* cp = P.colors + 3 * crow;
                 col[0] = cp[0]; col[1] = cp[1]; col[2] = cp[2];
             }
-            const ItemOut o = project_item(P, idx);
+            const ItemOut o = project_item(P, idx, bid);
             cnt[k] = o.count;
             if constexpr (kFused) {
                 float4 r[4];
                 pack_record(o.x, o.y, o.a, o.b, o.c, o.opac, P.compensate, col, o.depth, r);
-                float4* dst = P.recs + 4 * idx;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) dst[q] = r[q];
+                for (int q = 0; q < 4; ++q) s_rec[4 * tid + (q ^ ((tid >> 2) & 3))] = r[q];
                 // visible items (radii > 0) set the range, splax/_rasterize/_sort/_kernels.py:38-73;
-                // slot 0 or 1: with n >= kThreads a chunk meets at most two images
+                // slot 0 or 1: with n >= kProjChunk a chunk meets at most two images
                 if (P.mm_partial && o.count > 0) {
-                    const bool second = idx / P.n != base / P.n;
+                    const bool second = bid != (int32_t)item_quot(base, P.by_n);
                     const uint32_t u = f2ord(o.depth);
                     if (second) {
                         mm[2] = u;
@@ -280,8 +289,24 @@ __global__ void __launch_bounds__(kThreads) project_fwd_kernel(ProjectParams P) 
         }
         local += cnt[k];
     }
-    // block inclusive scan of `local`
     const int lane = tid & 63, wave = tid >> 6;
+    if constexpr (kFused) {
+        // Consecutive lanes store consecutive float4s: stored by its own lane, a record is four
+        // stores of 16 bytes at a stride of 64 (12M items 408 -> 402 us, 8M 227 -> 218 us, with
+        // workgroups of 1024).
+        __builtin_amdgcn_wave_barrier();
+        const int64_t first = base + wave * 64;
+        const int64_t left = P.total - first;
+        const int parts = 4 * (int)(left < 64 ? left : 64);  // negative for a wave past the end
+        const float4* src = s_rec + wave * 256;
+        float4* dst = P.recs + 4 * first;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int k = q * 64 + lane;
+            if (k < parts) dst[k] = src[k ^ ((k >> 4) & 3)];
+        }
+    }
+    // block inclusive scan of `local`
     int32_t incl = wave_inclusive_scan_i32(local, lane);
     if (lane == 63) s_wave[wave] = incl;
     if constexpr (kFused) {
@@ -324,114 +349,139 @@ __global__ void __launch_bounds__(kThreads) project_fwd_kernel(ProjectParams P) 
     }
 }
 
-// Exclusive scan of the chunk totals in place, one 1024-thread workgroup: each thread sums a
-// contiguous run of chunks, the runs are scanned in LDS, then each thread writes its run's
-// prefixes.
-constexpr int kChunkScanThreads = 1024;
-// Two independent single-workgroup passes between the projection and the sort, in one launch:
-// (1) block 0 (when chunks > 1) turns the chunk totals into exclusive prefixes, which
-//     chunk_offset_kernel (or, on the render path, the emission) then adds to the chunks' items,
-//     and with total_out non-null writes the grand total (the intersection count) there, and
-//     with total_host non-null also into that host-visible word under host_tag (one 64-bit
-//     system-scope store, which the host polls for: no copy launch and no event, whose barrier
-//     packet every forward paid for);
-// (2) with mm non-null, block b < images folds the fused projection's per-chunk depth-range
-//     partials of image b into the image's range of visible items (what minmax_partial_kernel /
-//     minmax_final_kernel give): chunk c holds items [chunk_items c, chunk_items (c + 1)), its
+// Per-launch work on the chunks:
+// (1) block 0 turns the chunk totals into exclusive prefixes, which chunk_offset_kernel (or, on
+//     the render path, the emission) then adds to the chunks' items, and with total_out non-null
+//     writes the grand total (the intersection count) there, and with total_host non-null also
+//     into that host-visible word under host_tag (one 64-bit system-scope store, which the host
+//     polls for: no copy launch and no event, whose barrier packet every forward paid for);
+// (2) with mm non-null, block 1 + b folds the fused projection's per-chunk depth-range partials of
+//     image b into the image's range of visible items (what minmax_partial_kernel /
+//     minmax_final_kernel give): chunk c holds items [kProjChunk c, kProjChunk (c + 1)), its
 //     slot 0 the image of its first item, slot 1 the next.
-// kChunkScanPer: chunks per thread kept in registers. The launch takes the smallest of 4, 16 and
-// 64 that holds the run (64 predicated loads for one chunk each cost half of the kernel: 6.3 us
-// at 10 to 400 chunks, 3.0 to 3.6 us with 4; 13.0 and 12.3 us at 12K chunks with 16).
-template <int kChunkScanPer>
+// The scan is one workgroup's latency: all its totals are loaded at once, four consecutive ones
+// per thread and span of 4096 (a run of consecutive chunks per thread, 184 bytes apart over the
+// lanes at 47K chunks, took 76 us there), then one scan over the waves' sums. kSpans: the launch
+// takes the smallest of 1, 4 and 12 that holds the chunks (2.5 us at 40 to 400 chunks, 4.7 at
+// 3.9K, 9 at 31K and 47K); longer rows go round again.
+constexpr int kChunkScanThreads = 1024;
+constexpr int kChunkScanSpan = 4 * kChunkScanThreads;
+template <int kSpans>
 __global__ void __launch_bounds__(kChunkScanThreads)
-chunk_scan_kernel(uint32_t* sums, int64_t chunks, int32_t chunk_items, const uint32_t* partial, int32_t n, float* mm,
-                  int64_t images, int32_t* total_out, uint64_t* total_host, uint32_t host_tag) {
-    __shared__ uint32_t s_wave[kChunkScanThreads / 64];
-    __shared__ uint32_t s_lo[kChunkScanThreads / 64], s_hi[kChunkScanThreads / 64];
+chunk_scan_kernel(uint32_t* sums, int64_t chunks, const uint32_t* partial, int32_t n, float* mm,
+                  int32_t* total_out, uint64_t* total_host, uint32_t host_tag) {
+    constexpr int kWaves = kChunkScanThreads / 64, kSums = kSpans * kWaves;
+    __shared__ uint32_t s_sum[kSums + 1];
+    __shared__ uint32_t s_lo[kWaves], s_hi[kWaves];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (blockIdx.x == 0 && chunks > 1) {
-        const int64_t per = (chunks + kChunkScanThreads - 1) / kChunkScanThreads;
-        const int64_t lo = (int64_t)tid * per;
-        const int64_t hi = lo + per < chunks ? lo + per : chunks;
-        // runs of up to kChunkScanPer chunks (up to 64Ki chunks, 67M items) are loaded into
-        // registers at once, so their load latencies overlap; longer runs take a sequential loop
-        const bool in_regs = per <= kChunkScanPer;
-        uint32_t v[kChunkScanPer];
-        uint32_t total = 0;
-        if (in_regs) {
+    if (blockIdx.x == 0) {
+        uint32_t carry = 0;
+        for (int64_t c0 = 0; c0 < chunks; c0 += (int64_t)kSpans * kChunkScanSpan) {
+            uint32_t v[kSpans][4], incl[kSpans];
 #pragma unroll
-            for (int k = 0; k < kChunkScanPer; ++k) v[k] = lo + k < hi ? sums[lo + k] : 0u;
+            for (int t = 0; t < kSpans; ++t) {
+                const int64_t c = c0 + t * kChunkScanSpan + 4 * tid;
+                if (c + 4 <= chunks) {
+                    const uint4 x = *reinterpret_cast<const uint4*>(sums + c);
+                    v[t][0] = x.x; v[t][1] = x.y; v[t][2] = x.z; v[t][3] = x.w;
+                } else {
 #pragma unroll
-            for (int k = 0; k < kChunkScanPer; ++k) total += v[k];
-        } else {
-            for (int64_t c = lo; c < hi; ++c) total += sums[c];
-        }
-        // exclusive prefix of the run totals: a wave scan, then the totals of the waves before
-        const uint32_t incl = (uint32_t)wave_inclusive_scan_i32((int32_t)total, lane);
-        if (lane == 63) s_wave[wave] = incl;
-        __syncthreads();
-        uint32_t run = incl - total;
-        for (int w = 0; w < wave; ++w) run += s_wave[w];
-        if (in_regs) {
-#pragma unroll
-            for (int k = 0; k < kChunkScanPer; ++k) {
-                if (lo + k < hi) sums[lo + k] = run;
-                run += v[k];
+                    for (int k = 0; k < 4; ++k) v[t][k] = c + k < chunks ? sums[c + k] : 0u;
+                }
             }
-        } else {
-            for (int64_t c = lo; c < hi; ++c) {
-                const uint32_t x = sums[c];
-                sums[c] = run;
-                run += x;
+#pragma unroll
+            for (int t = 0; t < kSpans; ++t) {
+                const uint32_t mine = (v[t][0] + v[t][1]) + (v[t][2] + v[t][3]);
+                incl[t] = (uint32_t)wave_inclusive_scan_i32((int32_t)mine, lane);
+                if (lane == 63) s_sum[t * kWaves + wave] = incl[t];
+                incl[t] -= mine;
             }
+            __syncthreads();
+            // exclusive scan of the waves' sums, in chunk order, by wave 0
+            if (wave == 0) {
+                constexpr int kPer = (kSums + 63) / 64;
+                uint32_t x[kPer], mine = 0;
+#pragma unroll
+                for (int k = 0; k < kPer; ++k) {
+                    x[k] = lane * kPer + k < kSums ? s_sum[lane * kPer + k] : 0u;
+                    mine += x[k];
+                }
+                const uint32_t end = (uint32_t)wave_inclusive_scan_i32((int32_t)mine, lane);
+                uint32_t run = end - mine;
+#pragma unroll
+                for (int k = 0; k < kPer; ++k) {
+                    if (lane * kPer + k < kSums) s_sum[lane * kPer + k] = run;
+                    run += x[k];
+                }
+                if (lane == 63) s_sum[kSums] = end;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int t = 0; t < kSpans; ++t) {
+                const int64_t c = c0 + t * kChunkScanSpan + 4 * tid;
+                uint32_t p[4];
+                p[0] = carry + s_sum[t * kWaves + wave] + incl[t];
+#pragma unroll
+                for (int k = 1; k < 4; ++k) p[k] = p[k - 1] + v[t][k - 1];
+                if (c + 4 <= chunks) {
+                    *reinterpret_cast<uint4*>(sums + c) = make_uint4(p[0], p[1], p[2], p[3]);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        if (c + k < chunks) sums[c + k] = p[k];
+                }
+            }
+            carry += s_sum[kSums];
+            __syncthreads();  // s_sum is written again by the next round
         }
-        // the last thread's run ends at the grand total (runs past the chunks are empty); int32
-        // wrap-around on overflow is kept, as in cum_tiles_hit
-        if (total_out && tid == kChunkScanThreads - 1) *total_out = (int32_t)run;
-        if (total_host && tid == kChunkScanThreads - 1)
-            __hip_atomic_store(total_host, ((uint64_t)host_tag << 32) | run, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-    if (mm != nullptr && (int64_t)blockIdx.x < images) {
-        const int64_t image = blockIdx.x;
-        const int64_t c0 = image * n / chunk_items;
-        int64_t c1 = ((image + 1) * n - 1) / chunk_items;
-        c1 = c1 < chunks - 1 ? c1 : chunks - 1;
-        uint32_t lo = 0xffffffffu, hi = 0u;
-        for (int64_t c = c0 + tid; c <= c1; c += kChunkScanThreads) {
-            const int64_t slot = image - c * chunk_items / n;  // 0 or 1
-            const uint32_t x = partial[4 * c + 2 * slot], y = partial[4 * c + 2 * slot + 1];
-            lo = x < lo ? x : lo;
-            hi = y > hi ? y : hi;
-        }
-        // the wave's range in lane 63 (DPP; every lane of the workgroup is here)
-        lo = wave_minmax_to_lane63<false>(lo);
-        hi = wave_minmax_to_lane63<true>(hi);
-        if (lane == 63) {
-            s_lo[wave] = lo;
-            s_hi[wave] = hi;
-        }
-        __syncthreads();
+        // int32 wrap-around on overflow is kept, as in cum_tiles_hit
         if (tid == 0) {
-            lo = 0xffffffffu;
-            hi = 0u;
-            for (int w = 0; w < kChunkScanThreads / 64; ++w) {
-                lo = s_lo[w] < lo ? s_lo[w] : lo;
-                hi = s_hi[w] > hi ? s_hi[w] : hi;
-            }
-            // no visible item: the reference's +-1e30 seeds remain (drange < 0 -> depth_q = 0)
-            mm[2 * image] = hi == 0u ? 1.0e30f : ord2f(lo);
-            mm[2 * image + 1] = hi == 0u ? -1.0e30f : ord2f(hi);
+            if (total_out) *total_out = (int32_t)carry;
+            if (total_host)
+                __hip_atomic_store(total_host, ((uint64_t)host_tag << 32) | carry,
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
+        return;
+    }
+    const int64_t image = (int64_t)blockIdx.x - 1, first = image * n;
+    const int64_t c0 = first >> kProjChunkShift;
+    int64_t c1 = (first + n - 1) >> kProjChunkShift;
+    c1 = c1 < chunks - 1 ? c1 : chunks - 1;
+    uint32_t lo = 0xffffffffu, hi = 0u;
+#pragma unroll 4
+    for (int64_t c = c0 + tid; c <= c1; c += kChunkScanThreads) {
+        const int64_t slot = c << kProjChunkShift < first;  // begins in the image before
+        const uint2 x = *reinterpret_cast<const uint2*>(partial + 4 * c + 2 * slot);
+        lo = x.x < lo ? x.x : lo;
+        hi = x.y > hi ? x.y : hi;
+    }
+    // the wave's range in lane 63 (DPP; every lane of the workgroup is here)
+    lo = wave_minmax_to_lane63<false>(lo);
+    hi = wave_minmax_to_lane63<true>(hi);
+    if (lane == 63) {
+        s_lo[wave] = lo;
+        s_hi[wave] = hi;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        lo = 0xffffffffu;
+        hi = 0u;
+        for (int w = 0; w < kWaves; ++w) {
+            lo = s_lo[w] < lo ? s_lo[w] : lo;
+            hi = s_hi[w] > hi ? s_hi[w] : hi;
+        }
+        // no visible item: the reference's +-1e30 seeds remain (drange < 0 -> depth_q = 0)
+        mm[2 * image] = hi == 0u ? 1.0e30f : ord2f(lo);
+        mm[2 * image + 1] = hi == 0u ? -1.0e30f : ord2f(hi);
     }
 }
 
 // cum_tiles_hit += the chunk's offset (chunk 0 has none); int32 wrap-around on overflow is kept,
 // the host reports a negative total as too many intersections. A chunk is one workgroup of the
 // projection and one of this kernel, one item per thread.
-__global__ void __launch_bounds__(kProjChunkBig) chunk_offset_kernel(int32_t* cum, int64_t total,
-                                                                     const uint32_t* offsets) {
-    const int64_t idx = (int64_t)(blockIdx.x + 1) * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(kProjChunk) chunk_offset_kernel(int32_t* cum, int64_t total,
+                                                                  const uint32_t* offsets) {
+    const int64_t idx = (int64_t)(blockIdx.x + 1) * kProjChunk + threadIdx.x;
     if (idx < total) cum[idx] = (int32_t)((uint32_t)cum[idx] + offsets[blockIdx.x + 1]);
 }
 
@@ -839,8 +889,7 @@ viewmat_reduce_kernel(const float* partials, int32_t blocks_per_image, float* v_
 
 // Chunks (workgroups) of a projection over `total` items: one chunk total of scratch each.
 int64_t project_fwd_chunks(int64_t total) {
-    const int64_t per_block = project_fwd_chunk_items(total);
-    return (total + per_block - 1) / per_block;
+    return (total + kProjChunk - 1) / kProjChunk;
 }
 
 int launch_project_fwd(const ProjectArgs& a, DeviceScratch& sc, hipStream_t stream) {
@@ -884,6 +933,11 @@ int launch_project_fwd_impl(const ProjectArgs& a, uint32_t* chunk_sums, const Fu
     P.total = a.total; P.img_h = a.img_h; P.img_w = a.img_w;
     P.fx = a.fx; P.fy = a.fy; P.cx = a.cx; P.cy = a.cy;
     P.glob_scale = a.glob_scale; P.clip_thresh = a.clip_thresh;
+    const float tan_fovx = 0.5f * (float)a.img_w / a.fx;
+    const float tan_fovy = 0.5f * (float)a.img_h / a.fy;
+    P.lim_x = kFovClamp * tan_fovx;
+    P.lim_y = kFovClamp * tan_fovy;
+    P.by_n = item_div(a.n, a.total);
     P.xys = a.xys; P.depths = a.depths; P.radii = a.radii; P.conics = a.conics;
     P.num_tiles_hit = a.num_tiles_hit; P.cum_tiles_hit = a.cum_tiles_hit;
     P.wxyz = a.quats_wxyz;
@@ -894,36 +948,28 @@ int launch_project_fwd_impl(const ProjectArgs& a, uint32_t* chunk_sums, const Fu
     P.mm_partial = f ? f->mm_partial : nullptr;
     // the render path leaves the chunk offsets to the emission when there are several chunks
     const bool offsets_later = f && f->count_word && blocks > 1;
-    const int32_t chunk = project_fwd_chunk_items(a.total);
-    const dim3 grid((unsigned)blocks), block(chunk);
-    if (f && chunk == kProjChunkSmall)
-        hipLaunchKernelGGL((project_fwd_kernel<true, kProjChunkSmall>), grid, block, 0, stream, P);
-    else if (f)
-        hipLaunchKernelGGL((project_fwd_kernel<true, kProjChunkBig>), grid, block, 0, stream, P);
-    else if (chunk == kProjChunkSmall)
-        hipLaunchKernelGGL((project_fwd_kernel<false, kProjChunkSmall>), grid, block, 0, stream, P);
+    const dim3 grid((unsigned)blocks), block(kProjChunk);
+    if (f)
+        hipLaunchKernelGGL(project_fwd_kernel<true>, grid, block, 0, stream, P);
     else
-        hipLaunchKernelGGL((project_fwd_kernel<false, kProjChunkBig>), grid, block, 0, stream, P);
+        hipLaunchKernelGGL(project_fwd_kernel<false>, grid, block, 0, stream, P);
     const int64_t images = (f && f->depth_mm) ? a.total / a.n : 0;
     if (blocks > 1 || images > 0) {
-        const dim3 scan_grid((unsigned)(images > 1 ? images : 1)), scan_block(kChunkScanThreads);
+        const dim3 scan_grid((unsigned)(1 + images)), scan_block(kChunkScanThreads);
         const uint32_t* mm_partial = f ? f->mm_partial : nullptr;
         float* mm = images > 0 ? f->depth_mm : nullptr;
         int32_t* count = offsets_later ? f->count_word : nullptr;
         uint64_t* host = offsets_later ? f->count_host : nullptr;
         const uint32_t tag = f ? f->count_tag : 0u;
-        if (blocks <= 4 * kChunkScanThreads)
+        if (blocks <= kChunkScanSpan)
+            hipLaunchKernelGGL(chunk_scan_kernel<1>, scan_grid, scan_block, 0, stream,
+                               P.chunk_sums, blocks, mm_partial, a.n, mm, count, host, tag);
+        else if (blocks <= 4 * kChunkScanSpan)
             hipLaunchKernelGGL(chunk_scan_kernel<4>, scan_grid, scan_block, 0, stream,
-                               P.chunk_sums, blocks, chunk, mm_partial, a.n, mm, images, count,
-                               host, tag);
-        else if (blocks <= 16 * kChunkScanThreads)
-            hipLaunchKernelGGL(chunk_scan_kernel<16>, scan_grid, scan_block, 0, stream,
-                               P.chunk_sums, blocks, chunk, mm_partial, a.n, mm, images, count,
-                               host, tag);
+                               P.chunk_sums, blocks, mm_partial, a.n, mm, count, host, tag);
         else
-            hipLaunchKernelGGL(chunk_scan_kernel<64>, scan_grid, scan_block, 0, stream,
-                               P.chunk_sums, blocks, chunk, mm_partial, a.n, mm, images, count,
-                               host, tag);
+            hipLaunchKernelGGL(chunk_scan_kernel<12>, scan_grid, scan_block, 0, stream,
+                               P.chunk_sums, blocks, mm_partial, a.n, mm, count, host, tag);
     }
     if (blocks > 1 && !offsets_later)
         return launch_chunk_offsets(P.cum_tiles_hit, a.total, P.chunk_sums, stream);
@@ -935,7 +981,7 @@ int launch_chunk_offsets(int32_t* cum, int64_t total, const uint32_t* chunk_pref
     const int64_t blocks = project_fwd_chunks(total);
     if (blocks > 1)
         hipLaunchKernelGGL(chunk_offset_kernel, dim3((unsigned)(blocks - 1)),
-                           dim3(project_fwd_chunk_items(total)), 0, stream, cum, total,
+                           dim3(kProjChunk), 0, stream, cum, total,
                            chunk_prefix);
     return hipGetLastError() == hipSuccess ? 0 : kErrLaunch;
 }
@@ -996,25 +1042,25 @@ int launch_project_bwd(const ProjectBwdArgs& a, DeviceScratch& sc, hipStream_t s
 }
 
 // ------------------------------------------------------------------ projection without allocation
-// splat_project_fwd_noalloc keeps its chunk totals in this fixed array of kNoAllocMaxChunks
+// splat_project_fwd_noalloc keeps its chunk totals in this fixed array of kNoAllocMaxItems / kProjChunk
 // uint32 (256 KiB), which each device the library runs on holds until the process ends. In host
 // code `scratch` names a host-side stand-in, not the device array: its device address comes from
 // hipGetSymbolAddress, once per device with that device current, and only that address is
 // passed to kernels. Every no-allocation call on a device shares the array, so such calls must
 // not overlap on one device (they would race on it); nothing in it needs to start at zero (the
 // projection writes every chunk total before the scan reads it).
-static __device__ __align__(256) uint32_t scratch[kNoAllocMaxChunks];
+static __device__ __align__(256) uint32_t scratch[kNoAllocMaxItems / kProjChunk];
 
 constexpr int kNoAllocDevices = 64;
 static std::mutex g_noalloc_mu;
 static uint32_t* g_noalloc_scratch[kNoAllocDevices] = {};
 
 int launch_project_fwd_noalloc(const ProjectArgs& a, hipStream_t stream) {
-    if (project_fwd_chunks(a.total) > kNoAllocMaxChunks)
+    if (a.total > kNoAllocMaxItems)
         return fail(kErrArgs, "project_fwd_noalloc: more than " +
-                                  std::to_string(kNoAllocMaxChunks * kProjChunkBig) +
-                                  " items (the fixed scratch holds " +
-                                  std::to_string(kNoAllocMaxChunks) + " chunk totals)");
+                                  std::to_string(kNoAllocMaxItems) +
+                                  " items (the fixed scratch holds one total per " +
+                                  std::to_string(kProjChunk) + ")");
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kNoAllocDevices)
         return fail(kErrRuntime, "project_fwd_noalloc: no usable current device");

@@ -231,8 +231,8 @@ int launch_project_fwd(const ProjectArgs& a, DeviceScratch& sc, hipStream_t stre
 int launch_project_fwd_into(const ProjectArgs& a, uint32_t* chunk_sums, hipStream_t stream);
 // The fused render forward's projection: also each item's packed blend record (recs, 4 float4
 // per item, from colors / compensate as launch_pack_records would write it) and, with depth_mm
-// non-null (requires n >= project_fwd_chunk_items), the per-image depth range of the visible items (mm_partial:
-// scratch of 4 uint32 per chunk), as the sort's depth-range kernels would compute it.
+// non-null (requires n >= kProjChunk), the per-image depth range of the visible items
+// (mm_partial: scratch of 4 uint32 per chunk), as the sort's depth-range kernels would compute it.
 struct FusedRecords {
     const float* colors; int64_t rows_colors;
     int32_t compensate;
@@ -252,16 +252,19 @@ int launch_project_fwd_fused(const ProjectArgs& a, const FusedRecords& f, Device
                              hipStream_t stream);
 int launch_project_fwd_impl(const ProjectArgs& a, uint32_t* chunk_sums, const FusedRecords* f,
                             hipStream_t stream);
-// Items per chunk of the projection's tile-count scan over `total` items (one projection workgroup
-// each, 256 or 1024 items), and the number of chunks.
-int32_t project_fwd_chunk_items(int64_t total);
+// Items per chunk of the projection's tile-count scan: one projection workgroup each, one item per
+// thread. A workgroup gives its CU's wave slots back when its slowest wave ends, and the ellipse
+// walks differ: with chunks of 1024 the projection took 433 us for 12M items, 235 us for 8M and
+// 40.9 us for 1M; with 256 it takes 367, 202 and 32.6 us, and 10K items are 40 workgroups instead
+// of 10 (6.5 us, 10.0 before).
+constexpr int kProjChunkShift = 8, kProjChunk = 1 << kProjChunkShift;
 int64_t project_fwd_chunks(int64_t total);
 // Adds chunk c's exclusive prefix to the items of chunk c, c >= 1.
 int launch_chunk_offsets(int32_t* cum, int64_t total, const uint32_t* chunk_prefix,
                          hipStream_t stream);
 // The projection with no allocation: its chunk totals in a fixed device array of
-// kNoAllocMaxChunks entries per device (one per 1024 items).
-constexpr int64_t kNoAllocMaxChunks = 65536;
+// kNoAllocMaxItems / kProjChunk entries per device.
+constexpr int64_t kNoAllocMaxItems = 65536 * 1024;
 int launch_project_fwd_noalloc(const ProjectArgs& a, hipStream_t stream);
 int launch_project_bwd(const ProjectBwdArgs& a, DeviceScratch& sc, hipStream_t stream);
 
