@@ -52,8 +52,8 @@ int splat_project_fwd(splat_stream_t stream, const float* means3d, int64_t rows_
 /* No counterpart in the reference: splat_project_fwd for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * Same arguments, validation and outputs as splat_project_fwd, bit for bit; the projection's
- * chunk-total scratch lives in a fixed device array of 65536 entries (256 KiB per device, held
- * until the process ends), so total is at most 65536 * 1024 = 67,108,864 items (status 1
+ * chunk-total scratch lives in a fixed device array of 262144 entries (1 MiB per device, held
+ * until the process ends), so total is at most 262144 * 256 = 67,108,864 items (status 1
  * beyond). It calls no allocating routine and uses none of the library's per-device scratch.
  * Every call on one device shares that array: calls that overlap on one device (different
  * streams or threads) race on it and must be serialized by the caller. */

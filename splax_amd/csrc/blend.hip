@@ -272,10 +272,10 @@ struct BlendFwdParams {
 // Bound by VALU issue, and by what the scalar unit and the branches add where a step's VALU do not
 // cover them. At most 64 VGPRs and 20480 bytes of LDS (no array beside the batch's: masks, wave
 // flags and loss sums take places that are free at the time), so eight waves per SIMD. At 1M
-// gaussians, 1920x1080: 163 us (153 with depth), at 8 views of 200K 430 us. Before: seven waves, a
+// gaussians, 1920x1080: 156 us (145 with depth), at 8 views of 200K 414 us. Before: seven waves, a
 // workgroup-wide count of done pixels per batch (three barriers), masks of 221 VALU, a flag for a
-// done pixel and both loop bounds in every step: 189, 189 and 498 us. The cheaper masks and the
-// one barrier alone were 181 with depth and 489 us, and the rest is the shorter step.
+// done pixel and both loop bounds in every step: 184, 190 and 500 us. The cheaper masks and the
+// one barrier alone were 181 with depth and 469 us, and the rest is the shorter step.
 template <bool kDepth>
 __global__ void __launch_bounds__(kTile, 8) blend_fwd_kernel(BlendFwdParams P) {
     __shared__ BatchLds<kTile> L;

@@ -254,9 +254,9 @@ int launch_project_fwd_impl(const ProjectArgs& a, uint32_t* chunk_sums, const Fu
                             hipStream_t stream);
 // Items per chunk of the projection's tile-count scan: one projection workgroup each, one item per
 // thread. A workgroup gives its CU's wave slots back when its slowest wave ends, and the ellipse
-// walks differ: with chunks of 1024 the projection took 433 us for 12M items, 235 us for 8M and
-// 40.9 us for 1M; with 256 it takes 367, 202 and 32.6 us, and 10K items are 40 workgroups instead
-// of 10 (6.5 us, 10.0 before).
+// walks differ: with chunks of 1024 the projection took 402 us for 12M items, 218 us for 8M and
+// 37.9 us for 1M; with 256 it takes 341, 183 and 30.5 us, and 10K items are 40 workgroups instead
+// of 10 (6.2 us, 10.0 before).
 constexpr int kProjChunkShift = 8, kProjChunk = 1 << kProjChunkShift;
 int64_t project_fwd_chunks(int64_t total);
 // Adds chunk c's exclusive prefix to the items of chunk c, c >= 1.
