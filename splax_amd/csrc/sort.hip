@@ -477,8 +477,8 @@ rts_scatter_kernel(const K* __restrict__ keys_in, const int32_t* __restrict__ va
                    const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ totals,
                    int64_t parts) {
     constexpr int kTile = kItems * kSortThreads;
-    static_assert(sizeof(KO) == sizeof(K) || (sizeof(K) == 4 && sizeof(KO) == 2),
-                  "narrowing writes a 32-bit key's high half");
+    static_assert(sizeof(KO) == sizeof(K) || 2 * sizeof(KO) == sizeof(K),
+                  "narrowing writes a key's high half");
     // one staging buffer carries keys, then positions, then ids (three rounds), so two
     // 1024-thread workgroups fit a CU's LDS at eight keys per thread
     constexpr int kStageWords = kTile * (sizeof(K) > 4 ? (int)(sizeof(K) / 4) : 1);
@@ -580,7 +580,7 @@ rts_scatter_kernel(const K* __restrict__ keys_in, const int32_t* __restrict__ va
             const uint32_t d = (uint32_t)(k >> shift) & 255u;
             dig[r >> 2] |= d << (8 * (r & 3));
             if constexpr (sizeof(KO) < sizeof(K))
-                keys_out[s_dest_base[d] + j] = (KO)(k >> 16);
+                keys_out[s_dest_base[d] + j] = (KO)(k >> (8 * sizeof(KO)));
             else
                 keys_out[s_dest_base[d] + j] = k;
         }
@@ -637,6 +637,28 @@ static void launch_pass(const K* keys_in, const int32_t* vals_in, const int32_t*
     hipLaunchKernelGGL((rts_scatter_kernel<K, kItems, KO>), dim3(segment_grid(parts)),
                        dim3(kSortThreads), 0, stream, keys_in, vals_in, ids_in, keys_out,
                        vals_out, ids_out, M, m_dev, shift, counts, totals, parts);
+}
+
+// One pass over 64-bit keys: kind 0 moves whole keys, 1 reads whole keys and writes their high
+// words, 2 moves high words (bits from 32 on). A pass is bound by what it moves per key, 40 bytes
+// of whole keys with both values or 28 of high words: the scatters of the six passes over 8 views'
+// keys 195 -> 173 us (32.5 us each, 29.0 for the fourth, 23.4 for the last two), their counts 56 ->
+// 53, the bin edges 12.3 -> 8.9.
+template <int kItems>
+static void wide_pass(int kind, const uint64_t* ki, const int32_t* vin, const int32_t* gi,
+                      uint64_t* ko, int32_t* vout, int32_t* iout, int64_t M, const int32_t* m_dev,
+                      int shift, uint32_t* pc, uint32_t* hist, int32_t* bins, int64_t nb2,
+                      hipStream_t stream) {
+    uint32_t* const high = reinterpret_cast<uint32_t*>(ko);
+    if (kind == 0)
+        launch_pass<uint64_t, kItems>(ki, vin, gi, ko, vout, iout, M, m_dev, shift, pc, hist, bins,
+                                      nb2, stream);
+    else if (kind == 1)
+        launch_pass<uint64_t, kItems, uint32_t>(ki, vin, gi, high, vout, iout, M, m_dev, shift, pc,
+                                                hist, bins, nb2, stream);
+    else
+        launch_pass<uint32_t, kItems>(reinterpret_cast<const uint32_t*>(ki), vin, gi, high, vout,
+                                      iout, M, m_dev, shift - 32, pc, hist, bins, nb2, stream);
 }
 
 // ------------------------------------------------------------------ small sorts
@@ -793,12 +815,14 @@ static void packed_pass(int kind, const void* ki, const int32_t* vin, const int3
 // kKind 2: _tile_bin_edges_64bit (splax/_rasterize/_sort/_kernels.py:244-269), the (image,
 // tile) field read from the high word; 0: the packed 32-bit key; 1: the packed key's high half
 // (bits 16-31: its image and tile fields, depth_bits >= 16).
-constexpr int kKeysPacked = 0, kKeysPackedHigh = 1, kKeysWide = 2;
+// 3: the 64-bit key's high word alone.
+constexpr int kKeysPacked = 0, kKeysPackedHigh = 1, kKeysWide = 2, kKeysWideHigh = 3;
 template <int kKind>
 __device__ __forceinline__ int32_t key_bin(const void* keys, int64_t i, int32_t num_tiles,
                                            int32_t tile_bits, int32_t depth_bits) {
-    if constexpr (kKind == kKeysWide) {
-        const uint64_t k = static_cast<const uint64_t*>(keys)[i] >> 32;
+    if constexpr (kKind >= kKeysWide) {
+        const uint64_t k = kKind == kKeysWide ? static_cast<const uint64_t*>(keys)[i] >> 32
+                                              : static_cast<const uint32_t*>(keys)[i];
         const uint64_t mask = ((uint64_t)1 << tile_bits) - 1;
         return (int32_t)(k >> tile_bits) * num_tiles + (int32_t)(k & mask);
     } else {
@@ -815,7 +839,7 @@ __device__ __forceinline__ int32_t key_bin(const void* keys, int64_t i, int32_t 
 // halves) or two (32-bit keys) where 4 scalar loads each took more load instructions than the
 // kernel's bytes (config 3's bins 18.6 -> 12.2 us); 4 wide keys.
 template <int kKind>
-constexpr int bin_keys() { return kKind == kKeysWide ? 4 : 8; }
+constexpr int bin_keys() { return kKind >= kKeysWide ? 4 : 8; }
 
 // The tile bin of key word w (kKind's layout).
 template <int kKind>
@@ -837,7 +861,7 @@ bin_edges_kernel(const void* keys, int64_t M_bound, const int32_t* m_dev, int32_
     const int64_t i0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * KB;
     if (i0 >= M) return;
     int32_t cur[KB];
-    if constexpr (kKind == kKeysWide) {
+    if constexpr (kKind >= kKeysWide) {
 #pragma unroll
         for (int k = 0; k < KB; ++k)
             cur[k] = i0 + k < M ? key_bin<kKind>(keys, i0 + k, num_tiles, tile_bits, depth_bits)
@@ -1064,6 +1088,9 @@ int run_sort_and_bin(const RasterInputs& in, DeviceScratch& sc, hipStream_t stre
             hipLaunchKernelGGL((emit_keys_kernel<false, false>), grid, dim3(256), 0, stream, E);
         if (hipGetLastError() != hipSuccess) return fail(kErrLaunch, "emit launch failed");
     }
+    // 64-bit keys beyond the small sort keep only their high words once the depth is sorted (four
+    // passes), unless the caller returns the keys
+    const bool wide_high = wide && !full_keys && M > kSortSmallM && ps.n > 4;
     {
         StageTimer tm(stream, kStageSort);
         const bool small = M <= kSortSmallM;
@@ -1139,14 +1166,16 @@ int run_sort_and_bin(const RasterInputs& in, DeviceScratch& sc, hipStream_t stre
                 continue;
             }
             if (wide) {
-                const uint64_t* ki = sc.wkeys[src];
-                uint64_t* ko = sc.wkeys[dst];
+                // wide_high: the last pass over the depth writes the keys' high words and the
+                // passes over the tile and image fields move those
                 if (big)
-                    launch_pass<uint64_t, 8>(ki, vin, sc.gids[src], ko, vout, iout, M, m_dev, shift,
-                                             sc.part_counts, sc.hist, bins, nb2, stream);
+                    wide_pass<8>(!wide_high || pass < 3 ? 0 : pass == 3 ? 1 : 2, sc.wkeys[src],
+                                 vin, sc.gids[src], sc.wkeys[dst], vout, iout, M, m_dev, shift,
+                                 sc.part_counts, sc.hist, bins, nb2, stream);
                 else
-                    launch_pass<uint64_t, 4>(ki, vin, sc.gids[src], ko, vout, iout, M, m_dev, shift,
-                                             sc.part_counts, sc.hist, bins, nb2, stream);
+                    wide_pass<4>(!wide_high || pass < 3 ? 0 : pass == 3 ? 1 : 2, sc.wkeys[src],
+                                 vin, sc.gids[src], sc.wkeys[dst], vout, iout, M, m_dev, shift,
+                                 sc.part_counts, sc.hist, bins, nb2, stream);
             } else {
                 // narrow: the pass over bits 8-15 writes the keys' high halves and the passes
                 // over bits 16-30 move 16-bit keys (the buffers hold either)
@@ -1184,7 +1213,10 @@ int run_sort_and_bin(const RasterInputs& in, DeviceScratch& sc, hipStream_t stre
         StageTimer tm(stream, kStageBins);
         const int kb = wide ? bin_keys<kKeysWide>() : bin_keys<kKeysPacked>();
         const dim3 grid((unsigned)((M + 256 * kb - 1) / (256 * kb)));
-        if (wide)
+        if (wide && wide_high)
+            hipLaunchKernelGGL(bin_edges_kernel<kKeysWideHigh>, grid, dim3(256), 0, stream, o.keys,
+                               M, m_dev, L.num_tiles, L.tile_bits, L.depth_bits, nbins, bins);
+        else if (wide)
             hipLaunchKernelGGL(bin_edges_kernel<kKeysWide>, grid, dim3(256), 0, stream, o.keys,
                                M, m_dev, L.num_tiles, L.tile_bits, L.depth_bits, nbins, bins);
         else if (narrow)
